@@ -11,6 +11,10 @@ flags=(--offload-arch=gfx950 -O3 -std=c++17 -fPIC
        -ffp-contract=off -fhip-fp32-correctly-rounded-divide-sqrt -fno-gpu-rdc
        -Xclang -target-feature -Xclang -packed-fp32-ops
        -Wall -Wno-unused-function -DCVK_SOURCE_HASH="${src_hash}")
+# Loop-invariant code motion on machine code is off for the day loops: it lifts the constants of the infect
+# kernels' double-precision polynomials out of their round loop into registers (172 vector registers against 90,
+# and spills under a bound), and the edge kernels lose 5 to 14 registers to the same.
+day_flags=(-mllvm -disable-machine-licm)
 sources=(cvk_mirror cvk_day cvk_batch cvk_relax cvk_popgen cvk_results cvk_clip cvk_diag cvk_sources)
 objdir="${here}/_build"
 mkdir -p "${objdir}"
@@ -18,7 +22,9 @@ pids=()
 objs=()
 for s in "${sources[@]}"; do
   rm -f "${objdir}/${s}.o"
-  "${HIPCC}" "${flags[@]}" -c "${here}/${s}.hip" -o "${objdir}/${s}.o" &
+  extra=()
+  case "${s}" in cvk_day|cvk_batch) extra=("${day_flags[@]}") ;; esac
+  "${HIPCC}" "${flags[@]}" "${extra[@]}" -c "${here}/${s}.hip" -o "${objdir}/${s}.o" &
   pids+=("$!")
   objs+=("${objdir}/${s}.o")
 done

@@ -287,8 +287,9 @@ struct BatchInfectArgs {
   const SegView* segs;    // [S * L]
   int32_t* log;
   int64_t log_capacity;
-  int32_t t, count_flows, allow_beds, n_variants;
+  int32_t t, count_flows, allow_beds, use_waning;
   uint32_t infect_blocks;      // workgroups [0, infect_blocks) infect; the rest resample day rs_t
+  int32_t words;               // touched words per wave and sweep (infect_words)
   uint32_t gen_mask;           // bit l: layer l's sources come from the resample stream of day t
   int32_t rs_t;
   int32_t n_rs_chunks;
@@ -296,8 +297,10 @@ struct BatchInfectArgs {
   const int64_t* rs_chunk_first;
 };
 
-// Occupancy hint 3 waves/SIMD, as for the single-sim infect pass: resample workgroups share the kernel.
-__global__ __launch_bounds__(INFECT_BLOCK, 3) void batch_infect_kernel(BatchCommon C, BatchInfectArgs ia) {
+// The single-sim infect pass over the concatenated agents: a target's sim comes from a binary search over the
+// agent offsets (LDS), done once, when its key is read. The flow counts of a wave's current sim gather in
+// LDS and go to the sim's row when the wave's targets (ascending) reach another sim, and at the end.
+__global__ __launch_bounds__(INFECT_BLOCK) void batch_infect_kernel(BatchCommon C, BatchInfectArgs ia) {
   if (blockIdx.x >= ia.infect_blocks) {  // the next day's resample
     batch_resample_chunks(C, ia.segs, ia.rs_chunk_seg, ia.rs_chunk_first, (int32_t)(blockIdx.x - ia.infect_blocks),
                           ia.n_rs_chunks, (int32_t)(gridDim.x - ia.infect_blocks), ia.rs_t, false);
@@ -305,24 +308,57 @@ __global__ __launch_bounds__(INFECT_BLOCK, 3) void batch_infect_kernel(BatchComm
   }
   __shared__ int32_t s_off[CVK_BATCH_MAX_SIMS + 1];  // agent offsets (total agents < 2^31)
   for (int j = threadIdx.x; j <= C.n_sims; j += INFECT_BLOCK) s_off[j] = (int32_t)ia.a_off[j];
+  __shared__ uint32_t s_count[INFECT_BLOCK / 64][64];  // N_INFECT_COLS used
+  static_assert(N_INFECT_COLS <= 64, "one lane per counter");
+  uint32_t* cnt = s_count[threadIdx.x >> 6];
+  cnt[lane_id()] = 0;
   __syncthreads();
   const int32_t t = ia.t;
-  __shared__ int32_t s_list[INFECT_BLOCK / 64][INFECT_WAVE_LIST];
+  __shared__ int32_t s_list[INFECT_BLOCK / 64][INFECT_LIST];
+  __shared__ InfectStage s_stage[INFECT_BLOCK / 64];
   int32_t* list = s_list[threadIdx.x >> 6];
+  InfectStage& stage = s_stage[threadIdx.x >> 6];
+  __shared__ LogStage s_log[INFECT_BLOCK / 64];
+  LogStage& records = s_log[threadIdx.x >> 6];
+  uint32_t n_log = 0;
+  const InfectStores stores = infect_stores(C.P, lane_id() & (INFECT_GROUP - 1));
   const int64_t n_words = (C.n_total + 31) / 32;
-  const int64_t stride = (int64_t)ia.infect_blocks * INFECT_BLOCK;
-  const int64_t n_sweeps = (n_words + stride - 1) / stride;
-  for (int64_t sw = 0; sw < n_sweeps; ++sw) {
-    const int64_t w = sw * stride + (int64_t)blockIdx.x * INFECT_BLOCK + threadIdx.x;
-    const uint32_t total = compact_touched(C.touched, w, n_words, C.n_total, list);
-    for (uint32_t base = 0; base < total; base += 64) {  // wave-uniform: one target per lane per round
-      InfectOut o = {KEY_NONE, false, false, false, false, 0u, 0u};
+  const int64_t stride = (int64_t)ia.infect_blocks * (INFECT_BLOCK / 64) * ia.words;
+  const bool has_word = (int32_t)lane_id() < ia.words;
+  int64_t w = ((int64_t)blockIdx.x * (INFECT_BLOCK / 64) + (threadIdx.x >> 6)) * ia.words + lane_id();
+  uint32_t bits = has_word && w < n_words ? gmem(C.touched)[w] : 0u;
+  int32_t cur = -1;  // the sim whose counts the wave holds
+  const auto flush = [&]() {
+    wave_sync_lds();
+    if (cur >= 0 && lane_id() < (uint32_t)N_INFECT_COLS && cnt[lane_id()])
+      atomicAdd(&C.results[((int64_t)cur * C.npts + t) * CVK_R_COLS + infect_col((int)lane_id())], cnt[lane_id()]);
+    cnt[lane_id()] = 0;
+    wave_sync_lds();
+  };
+  for (int64_t w0 = w - lane_id(); w0 < n_words; w0 += stride) {  // wave-uniform
+    const int64_t wn = w + stride;
+    const uint32_t next = has_word && wn < n_words ? gmem(C.touched)[wn] : 0u;
+    if (bits) gmem(C.touched)[w] = 0u;
+    const uint32_t total = compact_touched(bits, w, C.n_total, list);
+    w = wn;
+    bits = next;
+    for (uint32_t base = 0; base < total; base += 64) {  // wave-uniform
+      const uint32_t jl = base + lane_id();
+      const int32_t g = jl < total ? list[jl] : -1;
+      InfectIn x = {};
+      bool inf = false;
+      if (g >= 0) {
+        x = infect_load(C.P, C.winner, g, ia.use_waning != 0);
+        inf = infect_valid(x);
+        gmem(C.winner)[g] = KEY_NONE;
+      }
+      const uint64_t m = __ballot(inf);
+      if (!m) continue;
+      const uint32_t n_inf = (uint32_t)__popcll(m);
+      wave_sync_lds();  // the previous targets' groups are done with the stage
       int32_t source = -1, s = 0;
-      int64_t il = 0;
-      const uint32_t jj = base + lane_id();
-      const int32_t gi = jj < total ? list[jj] : -1;
-      if (gi >= 0) {
-        const int64_t g = gi;
+      const uint32_t l = key_layer(x.key);
+      if (inf) {
         int32_t lo = 0, hi = C.n_sims - 1;  // the sim with s_off[s] <= g < s_off[s + 1]
         while (lo < hi) {
           const int32_t mid = (lo + hi + 1) >> 1;
@@ -330,71 +366,54 @@ __global__ __launch_bounds__(INFECT_BLOCK, 3) void batch_infect_kernel(BatchComm
           else hi = mid - 1;
         }
         s = lo;
-        il = g - s_off[s];
         const cvk_params& prm = C.params[s];
-        const uint32_t* row = C.results + ((int64_t)s * C.npts + t) * CVK_R_COLS;
-        const bool hosp_max = ia.allow_beds && prm.n_beds_hosp >= 0 && (int64_t)row[CVK_R_MID_SEVERE] > prm.n_beds_hosp;
-        const bool icu_max = ia.allow_beds && prm.n_beds_icu >= 0 && (int64_t)row[CVK_R_MID_CRITICAL] > prm.n_beds_icu;
-        o = infect_target(C.P, prm, C.winner, g, (uint32_t)il, C.n_total, t, hosp_max, icu_max);
-        if (o.inf && (int32_t)o.l < C.n_layers) {
-          const SegView& L = ia.segs[s * C.n_layers + (int32_t)o.l];
-          source = key_source(o.key, L.p1, L.p2, (ia.gen_mask >> o.l) & 1u, prm.seed, t,
+        bool hosp_max = false, icu_max = false;
+        if (ia.allow_beds) {
+          const uint32_t* row = C.results + ((int64_t)s * C.npts + t) * CVK_R_COLS;
+          hosp_max = prm.n_beds_hosp >= 0 && (int64_t)row[CVK_R_MID_SEVERE] > prm.n_beds_hosp;
+          icu_max = prm.n_beds_icu >= 0 && (int64_t)row[CVK_R_MID_CRITICAL] > prm.n_beds_icu;
+        }
+        infect_stage(C.P, prm, stage, lanes_below(m), g, x, C.n_total, (uint32_t)s, hosp_max, icu_max);
+        if ((int32_t)l < C.n_layers && ia.log_capacity > 0) {  // the source is only for the log
+          const SegView& L = ia.segs[s * C.n_layers + (int32_t)l];
+          source = key_source(x.key, L.p1, L.p2, (ia.gen_mask >> l) & 1u, prm.seed, t,
                               (uint32_t)(s_off[s + 1] - s_off[s]));
         }
       }
-      // infection log, people.py:509-511 (indices within the sim, sim in bits 12+ of the last word)
-      const uint64_t m = __ballot(o.inf);
-      if (m) {
-        unsigned long long base = 0;
-        if (lane_id() == 0)
-          base = atomicAdd((unsigned long long*)&C.ctl[CVK_CTL_LOG_COUNT], (unsigned long long)__popcll(m));
-        base = __shfl(base, 0, 64);
-        if (o.inf) {
-          const unsigned long long pos = base + lanes_below(m);
-          if ((int64_t)pos < ia.log_capacity) {
-            int4 rec;
-            rec.x = source;
-            rec.y = (int32_t)il;
-            rec.z = t;
-            rec.w = (int32_t)(o.l | (o.v << 8) | ((uint32_t)s << 12));
-            ((int4*)ia.log)[pos] = rec;
-          } else {
-            C.ctl[CVK_CTL_LOG_OVERFLOW] = 1;
+      // indices within the sim, the sim in bits 12+
+      log_append(records, n_log, m, inf, source, g - s_off[s], l | (key_variant(x.key) << 8) | ((uint32_t)s << 12), t,
+                 ia.log, ia.log_capacity, C.ctl);
+      wave_sync_lds();
+      for (uint32_t r = 0; r < n_inf; r += 64 / INFECT_GROUP) {  // wave-uniform
+        const uint32_t j = r + lane_id() / INFECT_GROUP;
+        const bool act = j < n_inf;
+        const uint32_t jc = act ? j : r;
+        const uint32_t tag = stage.tag[jc];
+        const int32_t sj = (int32_t)(tag >> 8);
+        const cvk_params& prm = C.params[sj];
+        const auto dur_of = [&](int d) { return d < DUR_NAB ? prm.dur[d] : prm.nab_init; };
+        const InfectOut o = infect_group(prm, dur_of, stores, stage, jc, act, (uint32_t)(stage.g[jc] - s_off[sj]), t);
+        if (ia.count_flows) {
+          const int col = infect_count(o, tag & 0xFu);
+          bool pending = act;  // lanes peeled by sim
+          while (true) {
+            const uint64_t pm = __ballot(pending);
+            if (!pm) break;
+            const int32_t sl = __shfl(sj, __ffsll((unsigned long long)pm) - 1, 64);
+            if (sl != cur) {
+              flush();
+              cur = sl;
+            }
+            if (pending && sj == sl && col >= 0) atomicAdd(&cnt[col], 1u);
+            pending = pending && sj != sl;
           }
         }
-      }
-      // flows: lanes peeled by sim (targets of one sim are adjacent), one atomic per column per sim
-      bool pending = ia.count_flows && o.inf;
-      while (true) {
-        const uint64_t pm = __ballot(pending);
-        if (!pm) break;
-        const int lead = __ffsll((unsigned long long)pm) - 1;
-        const int32_t sl = __shfl(s, lead, 64);
-        const bool mine = pending && s == sl;
-        uint32_t cnt[N_INFECT_COLS];
-        cnt[0] = (uint32_t)__popcll(__ballot(mine));
-        cnt[1] = (uint32_t)__popcll(__ballot(mine && o.reinf));
-        for (int vv = 0; vv < MAXV; ++vv) {
-          if (vv < ia.n_variants) {
-            cnt[2 + vv] = (uint32_t)__popcll(__ballot(mine && o.v == (uint32_t)vv));
-            cnt[2 + MAXV + vv] = (uint32_t)__popcll(__ballot(mine && o.symp && o.v == (uint32_t)vv));
-            cnt[2 + 2 * MAXV + vv] = (uint32_t)__popcll(__ballot(mine && o.sev && o.v == (uint32_t)vv));
-          } else {
-            cnt[2 + vv] = cnt[2 + MAXV + vv] = cnt[2 + 2 * MAXV + vv] = 0;
-          }
-        }
-        if ((int)lane_id() == lead) {
-          uint32_t* row = C.results + ((int64_t)sl * C.npts + t) * CVK_R_COLS;
-          for (int k = 0; k < N_INFECT_COLS; ++k)
-            if (cnt[k]) atomicAdd(&row[infect_col(k)], cnt[k]);
-        }
-        pending = pending && !mine;
       }
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");  // the list is rewritten by the next sweep
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_sync_lds();  // the list is rewritten by the next sweep
   }
+  if (ia.count_flows) flush();
+  log_close(records, n_log, t, ia.log, ia.log_capacity, C.ctl);
 }
 
 // ---------------------------------------------------------------------------
@@ -829,12 +848,9 @@ static int launch_infect(Batch& b, int32_t t, int count_flows, hipStream_t st, i
   ia.t = t;
   ia.count_flows = count_flows;
   ia.allow_beds = count_flows;
-  ia.n_variants = b.V;
-  {  // as the single-sim infect pass: one sweep's workgroups, between one and three per CU
-    const int64_t n_cu = std::max(1, b.n_cu);
-    const int64_t want = (b.N / 32 + INFECT_BLOCK) / INFECT_BLOCK;
-    ia.infect_blocks = (uint32_t)std::min<int64_t>(std::max<int64_t>(want, n_cu), 3 * n_cu);
-  }
+  ia.use_waning = b.params[0].use_waning;  // the same for every sim
+  ia.infect_blocks = (uint32_t)infect_blocks_for(b.N, std::max(1, b.n_cu), 1 << 20);
+  ia.words = infect_words((b.N + 31) / 32, (int64_t)ia.infect_blocks * (INFECT_BLOCK / 64));
   uint32_t rs_blocks = 0;
   if (resample_t >= 0 && b.n_rs_chunks > 0) {
     ia.rs_t = resample_t;

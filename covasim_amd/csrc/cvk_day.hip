@@ -436,14 +436,13 @@ struct InfectArgs {
   uint32_t gen_mask;  // bit l: layer l's endpoints of day t come from the resample stream
   int32_t partial;    // 1: flow counts go to the infect partial rows (reduced later), 0: atomics on the row
   uint32_t infect_blocks;  // workgroups [0, infect_blocks) infect; the rest resample day rs_t
+  int32_t words;           // touched words per wave and sweep (infect_words)
   int32_t rs_t;
   int32_t n_resample;
   ResampleLayer rs[CVK_MAX_LAYERS];
 };
 
-// Occupancy hint 3 waves/SIMD (168 VGPRs, a few spills in the latency-bound outcome tree): the store-bound
-// resample workgroups sharing this kernel need the occupancy more than the infect lanes need registers.
-__global__ __launch_bounds__(INFECT_BLOCK, 3) void infect_pass_kernel(cvk_people P, cvk_params prm, cvk_work W,
+__global__ __launch_bounds__(INFECT_BLOCK) void infect_pass_kernel(cvk_people P, cvk_params prm, cvk_work W,
                                                                       InfectArgs ia) {
   if (blockIdx.x >= ia.infect_blocks) {  // the next day's resample, one thread per pair of edges
     const int64_t stride = (int64_t)(gridDim.x - ia.infect_blocks) * INFECT_BLOCK;
@@ -457,77 +456,74 @@ __global__ __launch_bounds__(INFECT_BLOCK, 3) void infect_pass_kernel(cvk_people
     return;
   }
   __shared__ uint32_t s_cnt[N_INFECT_COLS];
+  __shared__ cvk_dur s_dur[DUR_NAB + 1];
   if (threadIdx.x < N_INFECT_COLS) s_cnt[threadIdx.x] = 0;
+  if (threadIdx.x <= (unsigned)DUR_NAB) s_dur[threadIdx.x] = threadIdx.x < DUR_NAB ? prm.dur[threadIdx.x] : prm.nab_init;
   __syncthreads();
   const int32_t t = ia.t;
   const uint32_t* row = day_row(W, t);
   const bool hosp_max = ia.allow_beds && prm.n_beds_hosp >= 0 && (int64_t)row[CVK_R_MID_SEVERE] > prm.n_beds_hosp;
   const bool icu_max = ia.allow_beds && prm.n_beds_icu >= 0 && (int64_t)row[CVK_R_MID_CRITICAL] > prm.n_beds_icu;
-  // one touched-bitmap word (32 agents) per thread per sweep, compacted per wave into an LDS list;
-  // each round gives every lane one target
-  __shared__ int32_t s_list[INFECT_BLOCK / 64][INFECT_WAVE_LIST];
+  // Each wave takes ia.words touched words (32 agents each) per sweep, the next sweep's words loaded ahead, and
+  // compacts their targets into its LDS list; 64 at a time are staged, then eight at a time drawn and stored
+  __shared__ int32_t s_list[INFECT_BLOCK / 64][INFECT_LIST];
+  __shared__ InfectStage s_stage[INFECT_BLOCK / 64];
   int32_t* list = s_list[threadIdx.x >> 6];
+  InfectStage& stage = s_stage[threadIdx.x >> 6];
+  __shared__ LogStage s_log[INFECT_BLOCK / 64];
+  LogStage& records = s_log[threadIdx.x >> 6];
+  uint32_t n_log = 0;
+  const InfectStores stores = infect_stores(P, lane_id() & (INFECT_GROUP - 1));
+  const auto dur_of = [&](int d) { return s_dur[d]; };
   const int64_t n_words = (P.n + 31) / 32;
-  const int64_t stride = (int64_t)ia.infect_blocks * INFECT_BLOCK;
-  const int64_t n_sweeps = (n_words + stride - 1) / stride;
-  for (int64_t sw = 0; sw < n_sweeps; ++sw) {
-    const int64_t w = sw * stride + (int64_t)blockIdx.x * INFECT_BLOCK + threadIdx.x;
-    const uint32_t total = compact_touched(W.touched, w, n_words, P.n, list);
+  const int64_t stride = (int64_t)ia.infect_blocks * (INFECT_BLOCK / 64) * ia.words;
+  const bool has_word = (int32_t)lane_id() < ia.words;
+  int64_t w = ((int64_t)blockIdx.x * (INFECT_BLOCK / 64) + (threadIdx.x >> 6)) * ia.words + lane_id();
+  uint32_t bits = has_word && w < n_words ? gmem(W.touched)[w] : 0u;
+  for (int64_t w0 = w - lane_id(); w0 < n_words; w0 += stride) {  // wave-uniform
+    const int64_t wn = w + stride;
+    const uint32_t next = has_word && wn < n_words ? gmem(W.touched)[wn] : 0u;
+    if (bits) gmem(W.touched)[w] = 0u;
+    const uint32_t total = compact_touched(bits, w, P.n, list);
+    w = wn;
+    bits = next;
     for (uint32_t base = 0; base < total; base += 64) {  // wave-uniform
-      InfectOut o = {KEY_NONE, false, false, false, false, 0u, 0u};
-      int32_t source = -1, i = 0;
-      const uint32_t j = base + lane_id();
-      const int32_t g = j < total ? list[j] : -1;
-      if (g >= 0) {
-        i = g;
-        o = infect_target(P, prm, W.winner, i, (uint32_t)i, P.n, t, hosp_max, icu_max);
-        if (o.inf && (int32_t)o.l < ia.n_layers)
-          source = key_source(o.key, ia.p1[o.l], ia.p2[o.l], (ia.gen_mask >> o.l) & 1u, prm.seed, t, (uint32_t)P.n);
+      const uint32_t jl = base + lane_id();
+      const int32_t i = jl < total ? list[jl] : -1;
+      InfectIn x = {};
+      bool inf = false;
+      if (i >= 0) {
+        x = infect_load(P, W.winner, i, prm.use_waning != 0);
+        inf = infect_valid(x);
+        gmem(W.winner)[i] = KEY_NONE;
       }
-      // infection log, people.py:509-511: one wave-aggregated append per round
-      const uint64_t m = __ballot(o.inf);
-      if (m) {
-        unsigned long long base = 0;
-        if (lane_id() == 0)
-          base = atomicAdd((unsigned long long*)&W.ctl[CVK_CTL_LOG_COUNT], (unsigned long long)__popcll(m));
-        base = __shfl(base, 0, 64);
-        if (o.inf) {
-          const unsigned long long pos = base + lanes_below(m);
-          if ((int64_t)pos < W.log_capacity) {
-            int4 rec;
-            rec.x = source;
-            rec.y = i;
-            rec.z = t;
-            rec.w = (int32_t)(o.l | (o.v << 8));
-            ((int4*)W.log)[pos] = rec;
-          } else {
-            W.ctl[CVK_CTL_LOG_OVERFLOW] = 1;
-          }
-        }
+      const uint64_t m = __ballot(inf);
+      if (!m) continue;
+      const uint32_t n_inf = (uint32_t)__popcll(m);
+      wave_sync_lds();  // the previous targets' groups are done with the stage
+      int32_t source = -1;
+      const uint32_t l = key_layer(x.key);
+      if (inf) {
+        infect_stage(P, prm, stage, lanes_below(m), i, x, P.n, 0u, hosp_max, icu_max);
+        if ((int32_t)l < ia.n_layers)
+          source = key_source(x.key, ia.p1[l], ia.p2[l], (ia.gen_mask >> l) & 1u, prm.seed, t, (uint32_t)P.n);
       }
-      if (ia.count_flows && m) {
-        const uint32_t n_inf = (uint32_t)__popcll(m);
-        const uint32_t n_reinf = (uint32_t)__popcll(__ballot(o.inf && o.reinf));
-        if (lane_id() == 0) {
-          atomicAdd(&s_cnt[0], n_inf);
-          if (n_reinf) atomicAdd(&s_cnt[1], n_reinf);
-        }
-        for (int vv = 0; vv < prm.n_variants; ++vv) {
-          const uint32_t a0 = (uint32_t)__popcll(__ballot(o.inf && o.v == (uint32_t)vv));
-          const uint32_t a1 = (uint32_t)__popcll(__ballot(o.inf && o.symp && o.v == (uint32_t)vv));
-          const uint32_t a2 = (uint32_t)__popcll(__ballot(o.inf && o.sev && o.v == (uint32_t)vv));
-          if (lane_id() == 0) {
-            if (a0) atomicAdd(&s_cnt[2 + vv], a0);
-            if (a1) atomicAdd(&s_cnt[2 + MAXV + vv], a1);
-            if (a2) atomicAdd(&s_cnt[2 + 2 * MAXV + vv], a2);
-          }
+      log_append(records, n_log, m, inf, source, i, l | (key_variant(x.key) << 8), t, W.log, W.log_capacity, W.ctl);
+      wave_sync_lds();
+      for (uint32_t r = 0; r < n_inf; r += 64 / INFECT_GROUP) {  // wave-uniform
+        const uint32_t j = r + lane_id() / INFECT_GROUP;
+        const bool act = j < n_inf;
+        const uint32_t jc = act ? j : r;
+        const InfectOut o = infect_group(prm, dur_of, stores, stage, jc, act, (uint32_t)stage.g[jc], t);
+        if (ia.count_flows) {
+          const int col = infect_count(o, stage.tag[jc] & 0xFu);
+          if (col >= 0) atomicAdd(&s_cnt[col], 1u);
         }
       }
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");  // the list is rewritten by the next sweep
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_sync_lds();  // the list is rewritten by the next sweep
   }
+  log_close(records, n_log, t, W.log, W.log_capacity, W.ctl);
   __syncthreads();
   if (ia.count_flows && threadIdx.x < N_INFECT_COLS) {
     if (ia.partial)
@@ -1057,13 +1053,8 @@ static int infect_impl(const cvk_people* people, const cvk_layer* layers, const 
   ia.n_layers = params->n_layers;
   ia.count_flows = count_flows;
   ia.allow_beds = allow_beds;
-  // one touched-bitmap word per thread and sweep: enough workgroups for one sweep, at least one per CU and at
-  // most three (the occupancy the kernel's register budget allows), so large populations keep more waves
-  // in flight through the latency-bound outcome tree
-  const int n_cu = std::max(caps().n_cu, 1);
-  const int64_t want = (people->n / 32 + INFECT_BLOCK) / INFECT_BLOCK;
-  const int grid = (int)std::min<int64_t>(std::min<int64_t>(std::max<int64_t>(want, n_cu), 3 * (int64_t)n_cu),
-                                          INFECT_PART_BLOCKS);
+  const int grid = (int)infect_blocks_for(people->n, std::max(caps().n_cu, 1), INFECT_PART_BLOCKS);
+  ia.words = infect_words((people->n + 31) / 32, (int64_t)grid * (INFECT_BLOCK / 64));
   ia.partial = partial_blocks && count_flows ? 1 : 0;
   if (partial_blocks) *partial_blocks = ia.partial ? (uint32_t)grid : 0u;
   ia.infect_blocks = (uint32_t)grid;

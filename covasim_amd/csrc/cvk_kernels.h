@@ -1158,134 +1158,217 @@ __device__ inline void source_item_pass(const SimView& S, const SegView& L, cons
 }
 
 // ===========================================================================
-// People.infect for one target (people.py:470-579 + immunity.py:138-202)
+// People.infect (people.py:470-579 + immunity.py:138-202)
 // ===========================================================================
+// In two steps. First one lane per target: its key and every per-agent input in one memory round trip, the
+// branch probabilities, and the target's log record; the inputs go to the wave's LDS stage. Then eight
+// lanes per target, one per draw slot: the branch of the outcome tree is known to the whole group from the
+// two Bernoulli lanes, so the group needs one duration draw, executed once, where one lane per target runs
+// up to nine Philox + Box-Muller + exp chains one after another, one per duration of any branch some lane
+// of the wave takes (52 KB of code). Both steps of a wave without targets are empty. The draws, the
+// operations on them and so the results are those of the serial tree.
+constexpr int INFECT_BLOCK = 256;
+constexpr int INFECT_GROUP = 8;
+constexpr int INFECT_WORDS = 16;                 // touched words a wave takes per sweep, at most
+constexpr int INFECT_LIST = INFECT_WORDS * 32;   // every bit of them
+static_assert(SLOT_EXP2INF == 0 && SLOT_BERN_SYMP_SEV == 1 && SLOT_BERN_CRIT_DEATH == 2 && SLOT_DUR_A == 3 &&
+              SLOT_DUR_B == 4 && SLOT_DUR_C == 5 && SLOT_DUR_D == 6 && SLOT_NAB == 7, "one lane per draw slot");
+constexpr int DUR_NAB = 9;  // the peak-NAb distribution, after the nine durations
+
 struct InfectOut {
-  uint64_t key;  // the target's winning key (KEY_NONE: no infection)
   bool inf, reinf, symp, sev;
-  uint32_t v, l;
 };
 
-// g: storage index; il: index within the sim (counter field of the draws); stride: row stride of
-// the [variant][agent] arrays. Resets the target's winner key. The caller resolves the source.
-// Every per-agent input is loaded before the first store (the stores may alias the inputs for the
-// compiler, which would otherwise serialise one memory round trip per field).
-__device__ inline InfectOut infect_target(const cvk_people& P, const cvk_params& prm, uint64_t* winner, int64_t g,
-                                          uint32_t il, int64_t stride, int32_t t, bool hosp_max, bool icu_max) {
-  InfectOut o = {KEY_NONE, false, false, false, false, 0u, 0u};
-  const uint64_t key = winner[g];
-  const uint32_t f0 = P.flags[g];
-  o.key = key;
-  if (key == KEY_NONE || !(f0 & CVK_SUSCEPTIBLE)) {  // people.py:470 keeps susceptibles only
-    winner[g] = KEY_NONE;
-    return o;
+// The per-agent fields lane k of a group writes (every field is 4 bytes).
+struct InfectStores {
+  CVK_GLOBAL uint32_t *a, *b, *c;
+};
+__device__ inline InfectStores infect_stores(const cvk_people& P, uint32_t k) {
+  void *a, *b, *c;
+  switch (k) {
+    case 0: a = P.flags; b = P.date_critical; c = P.rel_trans; break;
+    case 1: a = P.vstate; b = P.date_diagnosed; c = P.n_breakthroughs; break;
+    case 2: a = P.n_infections; b = P.dur_disease; c = P.date_dead; break;
+    case 3: a = P.dur_exp2inf; b = P.date_recovered; c = P.t_nab_event; break;
+    case 4: a = P.date_exposed; b = P.dur_inf2sym; c = nullptr; break;
+    case 5: a = P.date_infectious; b = P.dur_sym2sev; c = nullptr; break;
+    case 6: a = P.date_symptomatic; b = P.dur_sev2crit; c = nullptr; break;
+    default: a = P.date_severe; b = P.peak_nab; c = nullptr; break;
   }
-  const uint32_t v = key_variant(key);
-  // inputs (one round trip)
-  const uint32_t vs0 = P.vstate[g];
-  const float peak0 = P.peak_nab[g];
-  const int32_t nb0 = P.n_breakthroughs[g];
-  const float rt0 = P.rel_trans[g];
-  const int32_t ninf0 = P.n_infections[g];
-  const float drec0 = P.date_recovered[g];
-  const float symp_p = P.symp_prob[g];
-  const float sev_p = P.severe_prob[g];
-  const float crit_p = P.crit_prob[g];
-  const float death_p = P.death_prob[g];
-  const float symp_imm = P.symp_imm[(int64_t)v * stride + g];
-  const float sev_imm = P.sev_imm[(int64_t)v * stride + g];
-  const float nab0 = prm.use_waning ? P.nab[g] : 0.0f;
-  winner[g] = KEY_NONE;
-  const uint64_t seed = prm.seed;
-  o.v = v;
-  o.l = key_layer(key);
-  o.inf = true;
-  // breakthrough, people.py:486-491
-  if (peak0 != 0.0f) {
-    if (nb0 == 0) P.rel_trans[g] = rt0 * prm.trans_redux;
-    P.n_breakthroughs[g] = nb0 + 1;
+  return InfectStores{gmem((uint32_t*)a), gmem((uint32_t*)b), gmem((uint32_t*)c)};
+}
+
+__device__ inline double shfl_d(double x, int src) {
+  const uint64_t u = (uint64_t)__double_as_longlong(x);
+  const uint32_t lo = (uint32_t)__shfl((int)(uint32_t)u, src, 64), hi = (uint32_t)__shfl((int)(uint32_t)(u >> 32), src, 64);
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+
+// The wave's stage: the inputs of up to 64 targets.
+struct InfectStage {
+  int32_t g[64];                           // storage index
+  uint32_t tag[64];                        // variant | reinfection << 4 | draws a new peak NAb << 5 | sim << 8
+  uint32_t f[64], vs[64];
+  float peak[64], rt[64];
+  int32_t nb[64], ninf[64];
+  float sp[64], sevp[64], critp[64], deathp[64];
+};
+
+// What one lane reads for its target, in one round trip (before any store: the stores may alias the inputs for
+// the compiler). The immunity rows are read for variant 0, the only one of most sims, until the key is here.
+struct InfectIn {
+  uint64_t key;
+  uint32_t f, vs;
+  float peak, rt, drec, symp, sev, crit, death, symp_imm, sev_imm, nab;
+  int32_t nb, ninf;
+};
+__device__ inline InfectIn infect_load(const cvk_people& P, const uint64_t* winner, int64_t g, bool waning) {
+  InfectIn x;
+  x.key = gmem(winner)[g];
+  x.f = gmem(P.flags)[g];
+  x.vs = gmem(P.vstate)[g];
+  x.peak = gmem(P.peak_nab)[g];
+  x.nb = gmem(P.n_breakthroughs)[g];
+  x.rt = gmem(P.rel_trans)[g];
+  x.ninf = gmem(P.n_infections)[g];
+  x.drec = gmem(P.date_recovered)[g];
+  x.symp = gmem(P.symp_prob)[g];
+  x.sev = gmem(P.severe_prob)[g];
+  x.crit = gmem(P.crit_prob)[g];
+  x.death = gmem(P.death_prob)[g];
+  x.symp_imm = gmem(P.symp_imm)[g];
+  x.sev_imm = gmem(P.sev_imm)[g];
+  x.nab = waning ? gmem(P.nab)[g] : 0.0f;
+  return x;
+}
+// The key names a susceptible target (people.py:470 keeps susceptibles only).
+__device__ inline bool infect_valid(const InfectIn& x) { return x.key != KEY_NONE && (x.f & CVK_SUSCEPTIBLE); }
+
+// Entry j of the stage from a valid target's inputs. stride: row stride of the [variant][agent] arrays.
+__device__ inline void infect_stage(const cvk_people& P, const cvk_params& prm, InfectStage& S, uint32_t j, int64_t g,
+                                    InfectIn x, int64_t stride, uint32_t sim, bool hosp_max, bool icu_max) {
+  const uint32_t v = key_variant(x.key);
+  if (v) {
+    x.symp_imm = gmem(P.symp_imm)[(int64_t)v * stride + g];
+    x.sev_imm = gmem(P.sev_imm)[(int64_t)v * stride + g];
   }
-  // states, people.py:494-506
-  P.flags[g] = (f0 & ~(CVK_SUSCEPTIBLE | CVK_NAIVE | CVK_RECOVERED | CVK_DIAGNOSED)) | CVK_EXPOSED;
-  P.vstate[g] = (vs0 & ~0xFu) | v | (1u << (8 + v));
-  P.n_infections[g] = ninf0 + 1;
-  o.reinf = !isnan(drec0);
-  // outcome tree, people.py:513-579
-  const float d_e2i = (float)draw_dur(prm.dur[CVK_DUR_EXP2INF], seed, il, t, SLOT_EXP2INF);
-  P.dur_exp2inf[g] = d_e2i;
-  P.date_exposed[g] = (float)t;
+  const bool new_peak = prm.use_waning && !(x.nab > 0.0f);
+  S.g[j] = (int32_t)g;
+  S.tag[j] = v | ((uint32_t)!isnan(x.drec) << 4) | ((uint32_t)new_peak << 5) | (sim << 8);
+  S.f[j] = x.f;
+  S.vs[j] = x.vs;
+  S.peak[j] = x.peak;
+  S.rt[j] = x.rt;
+  S.nb[j] = x.nb;
+  S.ninf[j] = x.ninf;
+  S.sp[j] = (prm.rel_symp_prob[v] * x.symp) * (1.0f - x.symp_imm);
+  S.sevp[j] = (prm.rel_severe_prob[v] * x.sev) * (1.0f - x.sev_imm);
+  S.critp[j] = (prm.rel_crit_prob[v] * x.crit) * (hosp_max ? prm.no_hosp_factor : 1.0f);
+  S.deathp[j] = (prm.rel_death_prob[v] * x.death) * (icu_max ? prm.no_icu_factor : 1.0f);
+}
+
+// Entry j of the stage by a group of eight lanes; every lane of the wave calls it (act is the same over a group,
+// j in range whether or not). il: index within the sim (counter field of the draws); dur_of(d): distribution
+// d (CVK_DUR_* or DUR_NAB).
+template <class DurOf>
+__device__ inline InfectOut infect_group(const cvk_params& prm, const DurOf& dur_of, const InfectStores& st,
+                                         const InfectStage& S, uint32_t j, bool act, uint32_t il, int32_t t) {
+  const uint32_t k = lane_id() & (INFECT_GROUP - 1);
+  const int lead = (int)(lane_id() & ~(uint32_t)(INFECT_GROUP - 1));
+  // this lane's slot
+  const u32x4 w = philox_seeded(prm.seed, il, (uint32_t)t, STREAM_INFECT, k);
+  const double u0 = u01(w.x, w.y), u1 = u01(w.z, w.w);
+  const double z = box_muller(u0, u1);
+  const double u_symp = shfl_d(u0, lead + (int)SLOT_BERN_SYMP_SEV), u_sev = shfl_d(u1, lead + (int)SLOT_BERN_SYMP_SEV);
+  const double u_crit = shfl_d(u0, lead + (int)SLOT_BERN_CRIT_DEATH), u_death = shfl_d(u1, lead + (int)SLOT_BERN_CRIT_DEATH);
+  // outcome, people.py:513-579
+  const uint32_t tag = S.tag[j];
+  const bool symp = u_symp < (double)S.sp[j];
+  const bool sev = symp && u_sev < (double)S.sevp[j];
+  const bool crit = sev && u_crit < (double)S.critp[j];
+  const bool death = crit && u_death < (double)S.deathp[j];
+  const bool new_peak = (tag >> 5) & 1u;
+  int d = CVK_DUR_EXP2INF;
+  bool need = act && k == SLOT_EXP2INF;
+  if (k == SLOT_DUR_A) { d = symp ? CVK_DUR_INF2SYM : CVK_DUR_ASYM2REC; need = act; }
+  if (k == SLOT_DUR_B) { d = sev ? CVK_DUR_SYM2SEV : CVK_DUR_MILD2REC; need = act && symp; }
+  if (k == SLOT_DUR_C) { d = crit ? CVK_DUR_SEV2CRIT : CVK_DUR_SEV2REC; need = act && sev; }
+  if (k == SLOT_DUR_D) { d = death ? CVK_DUR_CRIT2DIE : CVK_DUR_CRIT2REC; need = act && crit; }
+  if (k == SLOT_NAB) { d = DUR_NAB; need = act && new_peak; }
+  double dd = 0.0;
+  if (need) dd = sample_dur(dur_of(d), z, u0);
+  const double dd_e2i = shfl_d(dd, lead), dd_a = shfl_d(dd, lead + (int)SLOT_DUR_A), dd_b = shfl_d(dd, lead + (int)SLOT_DUR_B);
+  const double dd_c = shfl_d(dd, lead + (int)SLOT_DUR_C), dd_d = shfl_d(dd, lead + (int)SLOT_DUR_D);
+  const float d_e2i = (float)dd_e2i, d_i2s = (float)dd_a, d_s2s = (float)dd_b, d_s2c = (float)dd_c;
   const float date_inf = d_e2i + (float)t;
-  P.date_infectious[g] = date_inf;
+  const float date_sym = date_inf + d_i2s, date_sev = date_sym + d_s2s, date_crit = date_sev + d_s2c;
+  const float sum2 = d_e2i + d_i2s, sum3 = sum2 + d_s2s, sum4 = sum3 + d_s2c;
+  // the last duration of the branch, after the date and the disease time it starts from
+  const float from = !symp ? date_inf : !sev ? date_sym : !crit ? date_sev : date_crit;
+  const float before = !symp ? d_e2i : !sev ? sum2 : !crit ? sum3 : sum4;
+  const double last = !symp ? dd_a : !sev ? dd_b : !crit ? dd_c : dd_d;
+  const float end = (float)((double)from + last);
   const float fnan = __builtin_nanf("");
-  P.date_symptomatic[g] = fnan;
-  P.date_severe[g] = fnan;
-  P.date_critical[g] = fnan;
-  P.date_diagnosed[g] = fnan;
-  float date_rec = fnan;
-  double u_symp, u_sev, u_crit, u_death;
-  draw_pair(seed, il, t, SLOT_BERN_SYMP_SEV, u_symp, u_sev);
-  const float sp = (prm.rel_symp_prob[v] * symp_p) * (1.0f - symp_imm);
-  o.symp = u_symp < (double)sp;
-  int imm_class = 0;  // 0 asymptomatic, 1 mild, 2 severe (rel_imm_symp)
-  if (!o.symp) {
-    const double dd = draw_dur(prm.dur[CVK_DUR_ASYM2REC], seed, il, t, SLOT_DUR_A);
-    date_rec = (float)((double)date_inf + dd);
-    P.dur_disease[g] = (float)((double)d_e2i + dd);
-  } else {
-    const float d_i2s = (float)draw_dur(prm.dur[CVK_DUR_INF2SYM], seed, il, t, SLOT_DUR_A);
-    P.dur_inf2sym[g] = d_i2s;
-    const float date_sym = date_inf + d_i2s;
-    P.date_symptomatic[g] = date_sym;
-    const float sevp = (prm.rel_severe_prob[v] * sev_p) * (1.0f - sev_imm);
-    o.sev = u_sev < (double)sevp;
-    if (!o.sev) {
-      imm_class = 1;
-      const double dd = draw_dur(prm.dur[CVK_DUR_MILD2REC], seed, il, t, SLOT_DUR_B);
-      date_rec = (float)((double)date_sym + dd);
-      P.dur_disease[g] = (float)((double)(d_e2i + d_i2s) + dd);
-    } else {
-      imm_class = 2;
-      const float d_s2s = (float)draw_dur(prm.dur[CVK_DUR_SYM2SEV], seed, il, t, SLOT_DUR_B);
-      P.dur_sym2sev[g] = d_s2s;
-      const float date_sev = date_sym + d_s2s;
-      P.date_severe[g] = date_sev;
-      draw_pair(seed, il, t, SLOT_BERN_CRIT_DEATH, u_crit, u_death);
-      const float critp = (prm.rel_crit_prob[v] * crit_p) * (hosp_max ? prm.no_hosp_factor : 1.0f);
-      if (!(u_crit < (double)critp)) {
-        const double dd = draw_dur(prm.dur[CVK_DUR_SEV2REC], seed, il, t, SLOT_DUR_C);
-        date_rec = (float)((double)date_sev + dd);
-        P.dur_disease[g] = (float)((double)((d_e2i + d_i2s) + d_s2s) + dd);
-      } else {
-        const float d_s2c = (float)draw_dur(prm.dur[CVK_DUR_SEV2CRIT], seed, il, t, SLOT_DUR_C);
-        P.dur_sev2crit[g] = d_s2c;
-        const float date_crit = date_sev + d_s2c;
-        P.date_critical[g] = date_crit;
-        const float deathp = (prm.rel_death_prob[v] * death_p) * (icu_max ? prm.no_icu_factor : 1.0f);
-        const float dsum = ((d_e2i + d_i2s) + d_s2s) + d_s2c;
-        if (!(u_death < (double)deathp)) {
-          const double dd = draw_dur(prm.dur[CVK_DUR_CRIT2REC], seed, il, t, SLOT_DUR_D);
-          date_rec = (float)((double)date_crit + dd);
-          P.dur_disease[g] = (float)((double)dsum + dd);
-        } else {
-          const double dd = draw_dur(prm.dur[CVK_DUR_CRIT2DIE], seed, il, t, SLOT_DUR_D);
-          P.date_dead[g] = (float)((double)date_crit + dd);
-          P.dur_disease[g] = (float)((double)dsum + dd);
-        }
+  if (act) {
+    const float peak0 = S.peak[j];
+    const bool again = peak0 != 0.0f;  // breakthrough, people.py:486-491
+    uint32_t xa, xb = 0, xc = 0;
+    bool wb = true, wc = false;
+    switch (k) {
+      case 0:
+        xa = (S.f[j] & ~(CVK_SUSCEPTIBLE | CVK_NAIVE | CVK_RECOVERED | CVK_DIAGNOSED)) | CVK_EXPOSED;  // people.py:494-506
+        xb = __float_as_uint(crit ? date_crit : fnan);
+        xc = __float_as_uint(S.rt[j] * prm.trans_redux);
+        wc = again && S.nb[j] == 0;
+        break;
+      case 1:
+        xa = (S.vs[j] & ~0xFu) | (tag & 0xFu) | (1u << (8 + (tag & 0xFu)));
+        xb = __float_as_uint(fnan);  // date_diagnosed
+        xc = (uint32_t)(S.nb[j] + 1);
+        wc = again;
+        break;
+      case 2:
+        xa = (uint32_t)(S.ninf[j] + 1);
+        xb = __float_as_uint((float)((double)before + last));
+        xc = __float_as_uint(end);
+        wc = death;
+        break;
+      case 3:
+        xa = __float_as_uint(d_e2i);
+        xb = __float_as_uint(death ? fnan : end);
+        xc = (uint32_t)t;
+        wc = prm.use_waning != 0;
+        break;
+      case 4:
+        xa = __float_as_uint((float)t);
+        xb = __float_as_uint(d_i2s);
+        wb = symp;
+        break;
+      case 5:
+        xa = __float_as_uint(date_inf);
+        xb = __float_as_uint(d_s2s);
+        wb = sev;
+        break;
+      case 6:
+        xa = __float_as_uint(symp ? date_sym : fnan);
+        xb = __float_as_uint(d_s2c);
+        wb = crit;
+        break;
+      default: {  // update_peak_nab, immunity.py:138-202
+        xa = __float_as_uint(sev ? date_sev : fnan);
+        wb = prm.use_waning != 0;
+        const int imm_class = sev ? 2 : symp ? 1 : 0;  // asymptomatic, mild, severe (rel_imm_symp)
+        xb = __float_as_uint(new_peak ? (float)((pow(2.0, dd) * prm.rel_imm_symp[imm_class]) * prm.nab_norm)
+                                      : peak0 * prm.nab_boost);
+        break;
       }
     }
+    const int64_t g = S.g[j];
+    st.a[g] = xa;
+    if (wb) st.b[g] = xb;
+    if (wc) st.c[g] = xc;
   }
-  P.date_recovered[g] = date_rec;
-  // update_peak_nab, immunity.py:138-202
-  if (prm.use_waning) {
-    if (nab0 > 0.0f) {
-      P.peak_nab[g] = peak0 * prm.nab_boost;
-    } else {
-      const double init_nab = draw_dur(prm.nab_init, seed, il, t, SLOT_NAB);
-      P.peak_nab[g] = (float)((pow(2.0, init_nab) * prm.rel_imm_symp[imm_class]) * prm.nab_norm);
-    }
-    P.t_nab_event[g] = t;
-  }
-  return o;
+  return InfectOut{act, act && ((tag >> 4) & 1u), act && symp, act && sev};
 }
 
 // Source of an infection key (-1 for seeds and imports); p1/p2 are the sim's arrays of the key's layer.
@@ -1301,14 +1384,9 @@ __device__ inline int32_t key_source(uint64_t key, const int32_t* p1, const int3
   return key_dir(key) ? p2[e] : p1[e];
 }
 
-constexpr int INFECT_BLOCK = 256;
-constexpr int INFECT_WAVE_LIST = 64 * 32;  // every bit of one wave's 64 words
-
-// Compacts the set bits of this lane's touched word w (cleared in memory) into the wave's LDS list
-// `list` (storage indices, ascending lane order); returns the wave's total. All lanes call it.
-__device__ inline uint32_t compact_touched(uint32_t* touched, int64_t w, int64_t n_words, int64_t n, int32_t* list) {
-  uint32_t bits = w < n_words ? touched[w] : 0u;
-  if (bits) touched[w] = 0u;
+// Compacts the set bits of the lanes' touched words (bits, of word w) into the wave's LDS list `list` (storage
+// indices, ascending; -1 past the last agent); returns the wave's total. All lanes call it.
+__device__ inline uint32_t compact_touched(uint32_t bits, int64_t w, int64_t n, int32_t* list) {
   const uint32_t cnt = (uint32_t)__popc(bits);
   uint32_t incl = cnt;  // inclusive scan over the wave
 #pragma unroll
@@ -1324,12 +1402,109 @@ __device__ inline uint32_t compact_touched(uint32_t* touched, int64_t w, int64_t
     list[pos++] = g < n ? (int32_t)g : -1;
   }
   const uint32_t total = __shfl(incl, 63, 64);
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  wave_sync_lds();
   return total;
 }
+
+// Infection log records (people.py:509-511) wait in LDS, so that a workgroup makes one atomic on the log's
+// counter and not one per sweep of each wave: atomics on one address take ~9 ns each, and with one per
+// sweep the busy days of the 64-sim batch spent half their infect pass on them (632 against 314 us).
+constexpr int LOG_STAGE = 128;  // records a wave holds: fewer than 64 carried plus 64
+struct LogStage {
+  int32_t src[LOG_STAGE], tgt[LOG_STAGE];
+  uint32_t lv[LOG_STAGE];  // the record's last word: layer, variant, sim
+};
+
+// Writes the wave's n records from position pos of the log on.
+__device__ inline void log_write(const LogStage& L, uint32_t n, unsigned long long pos, int32_t t, int32_t* log,
+                                 int64_t capacity, uint32_t* ctl) {
+  for (uint32_t j = lane_id(); j < n; j += 64) {
+    if ((int64_t)(pos + j) < capacity) {
+      int4 rec;
+      rec.x = L.src[j];
+      rec.y = L.tgt[j];
+      rec.z = t;
+      rec.w = (int32_t)L.lv[j];
+      ((int4*)log)[pos + j] = rec;
+    } else {
+      ctl[CVK_CTL_LOG_OVERFLOW] = 1;
+    }
+  }
+}
+__device__ inline unsigned long long log_reserve(uint32_t* ctl, uint32_t n) {
+  return atomicAdd((unsigned long long*)&ctl[CVK_CTL_LOG_COUNT], (unsigned long long)n);
+}
+
+// Adds this lane's record (m: the lanes that have one) to the wave's stage, which is written out first when it
+// has no room. n: the records it holds.
+__device__ inline void log_append(LogStage& L, uint32_t& n, uint64_t m, bool mine, int32_t src, int32_t tgt, uint32_t lv,
+                                  int32_t t, int32_t* log, int64_t capacity, uint32_t* ctl) {
+  const uint32_t k = (uint32_t)__popcll(m);
+  if (n + k > (uint32_t)LOG_STAGE) {
+    unsigned long long pos = 0;
+    if (lane_id() == 0) pos = log_reserve(ctl, n);
+    pos = __shfl(pos, 0, 64);
+    wave_sync_lds();
+    log_write(L, n, pos, t, log, capacity, ctl);
+    wave_sync_lds();
+    n = 0;
+  }
+  if (mine) {
+    const uint32_t j = n + lanes_below(m);
+    L.src[j] = src;
+    L.tgt[j] = tgt;
+    L.lv[j] = lv;
+  }
+  n += k;
+}
+
+// The workgroup's remaining records, one reservation for all its waves (block-wide).
+__device__ inline void log_close(const LogStage& L, uint32_t n, int32_t t, int32_t* log, int64_t capacity, uint32_t* ctl) {
+  __shared__ uint32_t s_n[INFECT_BLOCK / 64];
+  __shared__ unsigned long long s_pos;
+  const uint32_t wave = threadIdx.x >> 6;
+  if (lane_id() == 0) s_n[wave] = n;
+  __syncthreads();
+  uint32_t before = 0, total = 0;
+  for (uint32_t k = 0; k < INFECT_BLOCK / 64; ++k) {
+    if (k < wave) before += s_n[k];
+    total += s_n[k];
+  }
+  if (total == 0) return;  // the same for the whole block
+  if (threadIdx.x == 0) s_pos = log_reserve(ctl, total);
+  __syncthreads();
+  log_write(L, n, s_pos + before, t, log, capacity, ctl);
+}
+
+// Touched words per wave and sweep: as few as one sweep over n_words by n_waves waves needs, so that every
+// wave has targets before any has many (the targets of one wave are served eight at a time).
+__host__ __device__ inline int32_t infect_words(int64_t n_words, int64_t n_waves) {
+  const int64_t w = (n_words + n_waves - 1) / n_waves;
+  return (int32_t)(w < 1 ? 1 : w > INFECT_WORDS ? INFECT_WORDS : w);
+}
+// Workgroups of an infect pass over n agents: enough for one sweep of INFECT_WORDS words a wave, at least one
+// per CU and at most three, and at most `most`.
+__host__ inline int64_t infect_blocks_for(int64_t n, int64_t n_cu, int64_t most) {
+  const int64_t per_block = (INFECT_BLOCK / 64) * INFECT_WORDS;
+  int64_t b = ((n + 31) / 32 + per_block - 1) / per_block;
+  b = b < n_cu ? n_cu : b > 3 * n_cu ? 3 * n_cu : b;
+  return b < most ? b : most;
+}
+
 constexpr int N_INFECT_COLS = 2 + 3 * MAXV;
+
+// The counter this lane of a target's group adds one to (infections, reinfections, then infections,
+// symptomatic and severe by variant), or -1.
+__device__ inline int infect_count(const InfectOut& o, uint32_t v) {
+  switch (lane_id() & (INFECT_GROUP - 1)) {
+    case 0: return o.inf ? 0 : -1;
+    case 1: return o.reinf ? 1 : -1;
+    case 2: return o.inf ? 2 + (int)v : -1;
+    case 3: return o.symp ? 2 + MAXV + (int)v : -1;
+    case 4: return o.sev ? 2 + 2 * MAXV + (int)v : -1;
+    default: return -1;
+  }
+}
 
 // Column of the day row for infect-pass counter k.
 __device__ inline int infect_col(int k) {

@@ -46,3 +46,18 @@ def test_boundary_run_matches_oracle(gpu, name, use_graph):
     assert_people_equal(sim, osim)
     if name in ('no_seeds', 'no_contacts'):
         assert sim.results['new_infections'].values.sum() == 0
+
+
+@pytest.mark.parametrize('n,k', [(33, 1), (33, 33), (2000, 9), (2000, 65), (200_003, 130_000), (200_003, 200_003)])
+def test_infection_counts_per_wave_match_oracle(gpu, n, k):
+    """Seeds only: from one target in the whole run to every agent of a wave's words (more than its log stage
+    holds); outcomes, counts and the log against the oracle."""
+    from tests.test_gpu_parity import assert_people_equal, assert_results_equal, run_pair
+    print(f'{k} seeds among {n}', flush=True)
+    pop = make_population(n=n, pop_type='random', contacts={'a': 0})
+    sim, osim, ores = run_pair(copy_pop(pop), n_days=1, seed=5, pop_type='random', use_waning=True, pop_infected=k)
+    assert_results_equal(sim, ores)
+    assert_people_equal(sim, osim)
+    log = sim.infection_log()
+    assert sorted(r['target'] for r in log) == sorted(tg for (_, tg, _, _, _) in osim.people.infection_log)
+    assert len(log) == k and all(r['source'] is None and r['layer'] == 'seed_infection' for r in log)
