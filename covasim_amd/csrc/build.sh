@@ -23,7 +23,7 @@ objs=()
 for s in "${sources[@]}"; do
   rm -f "${objdir}/${s}.o"
   extra=()
-  case "${s}" in cvk_day|cvk_batch) extra=("${day_flags[@]}") ;; esac
+  case "${s}" in cvk_day|cvk_batch|cvk_relax) extra=("${day_flags[@]}") ;; esac
   "${HIPCC}" "${flags[@]}" "${extra[@]}" -c "${here}/${s}.hip" -o "${objdir}/${s}.o" &
   pids+=("$!")
   objs+=("${objdir}/${s}.o")

@@ -804,11 +804,14 @@ typedef struct {
   int64_t n_agents;
   int32_t n_layers, n_days;
   int32_t kernel_len;          /* lags 0..kernel_len-1 of w_host per age bin */
-  int32_t checkpoint_every;    /* days between stored states (the backward re-runs each segment) */
+  int32_t checkpoint_every;    /* days between stored states where every day's record does not fit (the backward
+                                  then re-runs each segment) */
   int32_t precision;           /* 32 (float arithmetic) or 64 (double) */
-  int32_t pad;
+  int32_t segment_days;        /* 0: every day's record is held when half of the free memory takes them, else
+                                  checkpoint_every days; > 0: this many days. No result depends on it */
   double seed_frac;            /* pop_infected / n_agents */
-  const int64_t* indptr[CVK_MAX_LAYERS];  /* device [n_agents + 1]: neighbour list offsets per layer */
+  const int64_t* indptr[CVK_MAX_LAYERS];  /* device [n_agents + 1]: neighbour list offsets per layer (the lists
+                                             are laid out anew at create and not read afterwards) */
   const int32_t* nbr[CVK_MAX_LAYERS];     /* device: both directions of every edge, no self-loops */
   const uint8_t* age_bin;      /* device [n_agents]: prognosis age bin 0..9 */
   const float* rel_trans;      /* device [n_agents] */

@@ -346,3 +346,97 @@ def test_relax_calibration_reduces_loss_against_the_stochastic_curve(gpu):
     start = truth * np.random.default_rng(8).uniform(0.6, 1.5, relax.n_params)
     fitted, hist = calibrate(relax, observed, start, iters=80, lr=0.05)
     assert hist[-1] < 0.2 * hist[0], hist[::10]
+
+
+def _handle(relax, **fields):
+    """A second C handle over a Relaxation's descriptor with some of its fields replaced."""
+    import ctypes as C
+    from covasim_amd import _lib
+    d = _lib.RelaxDesc.from_buffer_copy(relax._desc)
+    for k, v in fields.items():
+        setattr(d, k, v)
+    h = C.c_void_p()
+    _lib.check(_lib.lib().cvk_relax_create(C.byref(d), C.byref(h)), 'cvk_relax_create')
+    return h
+
+
+def _value_and_grad(h, theta, c):
+    from covasim_amd import _lib
+    e, g = np.zeros(len(c)), np.zeros(len(theta))
+    L = _lib.lib()
+    try:
+        _lib.check(L.cvk_relax_forward(h, theta.ctypes.data, e.ctypes.data, _lib.stream_ptr()), 'forward')
+        _lib.check(L.cvk_relax_backward(h, theta.ctypes.data, c.ctypes.data, g.ctypes.data, _lib.stream_ptr()), 'backward')
+    finally:
+        _lib.check(L.cvk_relax_destroy(h), 'destroy')
+    return e, g
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('precision', [32, 64])
+@pytest.mark.parametrize('n', [63, 64, 65, 4001, 150_001])  # one agent short of, at and past a workgroup; both widths
+def test_relax_ragged_lists_match_cpu_reference(gpu, n, precision):
+    """A layer of one contact, a hub whose list goes through the stage in pieces, saturated contacts, agents without contacts;
+    records of all days or of segments give the same bits. Tolerances: each day adds a few roundings of the state
+    (2^-24 or 2^-53) and T = 12 days multiply them, some 50 in all, bounded here by 100."""
+    import torch
+    import covasim_amd as cv
+    from covasim_amd.relax import Relaxation
+    from tests.helpers import make_population
+    pop = make_population(n=n, seed=2, pop_type='hybrid')
+    hub = np.arange(1, min(n, 9000), dtype=np.int32)
+    for key, (a, b) in dict(h=(hub[:1], hub[1:2]), s=(np.zeros(len(hub), np.int32), hub)).items():
+        pop['contacts'][key] = dict(p1=a.copy(), p2=b.copy(), beta=np.ones(len(a), np.float32))
+    sim = cv.Sim(pop_size=n, pop_type='hybrid', n_days=12, rand_seed=3, popdict=pop, use_waning=False,
+                 dynam_layer=dict(c=1) if n % 2 else {}, pop_infected=min(20, n // 4)).initialize()
+    relax = Relaxation(sim, precision=precision, w_samples=5000)
+    theta = relax.theta0() * np.linspace(0.8, 1.2, relax.n_params)
+    theta[0] = 0.3  # the strongest transmitters' household-rate contacts saturate
+    csr, bins, rt, w, T, f, dyn = _cpu_inputs(relax)
+    c = np.random.default_rng(4).uniform(0.5, 1.5, T)
+    th = torch.tensor(theta, requires_grad=True)
+    e_ref = relax_ref.expected_infections(th, csr, bins, rt, w, T, f, dyn)
+    (torch.as_tensor(c) * e_ref).sum().backward()
+    tol = 100 * (2.0 ** -24 if precision == 32 else 2.0 ** -53)
+    whole = _value_and_grad(_handle(relax), theta, c)
+    assert _rel(whole[0], e_ref.detach().numpy()) <= tol
+    assert _rel(whole[1], th.grad.numpy()) <= tol
+    for days in (1, 5, 12):
+        part = _value_and_grad(_handle(relax, segment_days=days), theta, c)
+        assert np.array_equal(part[0], whole[0]) and np.array_equal(part[1], whole[1]), days
+
+
+@pytest.mark.gpu
+def test_relax_more_agents_than_a_packed_slot_addresses(gpu):
+    """2^25 + 3 agents (a slot's layer and bin then travel beside its index), contacts among the last few only: the
+    expected infections and gradient are those of the same few agents alone."""
+    import ctypes as C
+    import torch
+    from covasim_amd import _lib
+    few, T = 6, 5
+    pairs = np.array([(a, b) for a in range(few) for b in range(few) if a != b])
+    w = np.zeros((10, T + 1))
+    w[:, 1:] = np.random.default_rng(1).uniform(0.2, 1.5, (10, T))
+    theta = np.concatenate([[0.1, 1.3], np.linspace(0.5, 1.5, 10)])
+    c = np.linspace(1, 2, T)
+    out = []
+    for n in (few, 2 ** 25 + 3):
+        deg = torch.zeros(n, dtype=torch.int64, device='cuda')
+        deg[n - few:] = few - 1
+        indptr = torch.zeros(n + 1, dtype=torch.int64, device='cuda')
+        indptr[1:] = torch.cumsum(deg, 0)
+        nbr = torch.as_tensor(pairs[:, 1] + (n - few), dtype=torch.int32, device='cuda')
+        bins = torch.zeros(n, dtype=torch.uint8, device='cuda')
+        bins[n - few:] = torch.arange(few, dtype=torch.uint8, device='cuda') + 2
+        rt = torch.ones(n, dtype=torch.float32, device='cuda')
+        wh = np.ascontiguousarray(w)
+        d = _lib.RelaxDesc(n_agents=n, n_layers=1, n_days=T, kernel_len=T + 1, checkpoint_every=2, precision=32,
+                           seed_frac=0.05, age_bin=bins.data_ptr(), rel_trans=rt.data_ptr(), w_host=wh.ctypes.data)
+        d.indptr[0], d.nbr[0] = indptr.data_ptr(), nbr.data_ptr()
+        h = C.c_void_p()
+        _lib.check(_lib.lib().cvk_relax_create(C.byref(d), C.byref(h)), 'cvk_relax_create')
+        out.append(_value_and_grad(h, theta, c))
+    # the two sizes share an agent's products between different numbers of lanes, so a day's state may round the other
+    # way (2^-24); T = 5 days of a few such roundings, bounded as in the ragged cases
+    assert _rel(out[1][0], out[0][0]) <= 100 * 2.0 ** -24
+    assert _rel(out[1][1], out[0][1]) <= 100 * 2.0 ** -24
