@@ -295,6 +295,10 @@ def lib():
     L.cvk_infections.argtypes = [f32, vp, vp, vp, i64, vp, vp, i64, vp, u64, i32, i32, i32, i32, vp, vp, vp, i64,
                                  C.POINTER(C.c_int64), vp]
     L.cvk_infections_noalloc.argtypes = L.cvk_infections.argtypes
+    L.cvk_infections_work.argtypes = L.cvk_infections.argtypes[:-1] + [C.POINTER(i32), vp, i64, vp]
+    L.cvk_infections_work.restype = C.c_int
+    L.cvk_infections_work_bytes.argtypes = [i64, i64]
+    L.cvk_infections_work_bytes.restype = i64
     P, Pa, W, Ly = C.POINTER(PeopleS), C.POINTER(Params), C.POINTER(WorkS), C.POINTER(LayerS)
     L.cvk_choose.argtypes = [P, Pa, W, i32, u32, i64, i32, i32, i32, vp]
     L.cvk_agent_pass.argtypes = [P, Pa, W, i32, vp]

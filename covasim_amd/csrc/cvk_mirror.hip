@@ -3,6 +3,7 @@
 // output order. The production day loop (cvk_day.hip) fuses these steps.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "cvk_device.h"
@@ -58,7 +59,19 @@ __global__ void trans_sus_kernel(const float* __restrict__ rel_trans, const floa
   rs_out[i] = rs;
 }
 
-// utils.py:114-127: slot s in [0, n_dirs*E) is (direction s / E, edge s % E).
+// ---------------------------------------------------------------------------
+// compute_infections (utils.py:93-128): the transmitting pairs, direction by direction, edges ascending.
+//
+// Three launches. infections_bits: one bit per agent, rel_trans != 0. infections_scan: every wave takes a run of
+// 512-edge chunks; an edge is a candidate if the source of either of its directions has its bit set, and a chunk's
+// candidates, compacted in LDS, gather their factors and draw their uniform 64 at a time; one hit bit per
+// (direction, edge) and the waves' counts are kept. infections_write: each wave, from the sum of the counts before
+// its own, writes out its set bits. Reading the two endpoint columns once is what bounds the scan (80 MB and 20M
+// bit lookups at 10M edges, the bitmap in LDS up to ~1.1M agents); before, both a counting and a writing pass
+// gathered rel_trans at both ends of every edge and drew a Philox block per slot with a nonzero source, with one
+// workgroup scanning the counts between them: 129 + 149 + 21 us at 1M agents and 10M edges, 5 % of them
+// infectious, against 4 + 50 + 15 us. (The next chunk's columns loaded ahead of the candidates: 55 us.)
+// ---------------------------------------------------------------------------
 struct InfArgs {
   float beta;
   const int32_t* p1;
@@ -70,118 +83,247 @@ struct InfArgs {
   const double* uniforms;
   uint64_t seed;
   int32_t t, variant, layer;
-  int64_t n_slots;
+  int32_t dirs;        // 1 (legacy) or 2
+  int64_t n_agents;
+  // scratch
+  uint64_t* bits;      // one bit per agent, 16-byte aligned and padded (null: rel_trans itself is gathered)
+  int32_t lds_words;   // 32-bit words of it staged in LDS, or 0: read from memory
+  int64_t chunks;
+  uint32_t* hits;      // [2][chunks][16] hit bits
+  uint32_t* cnt;       // [2][waves] hits of each wave
+  uint64_t* out;       // [2] the total, and nonzero if an endpoint is outside [0, n_agents)
 };
 
-__device__ inline bool slot_transmits(const InfArgs& a, int64_t s, int32_t& src, int32_t& tgt, float& p) {
-  const int dir = s >= a.n_edges ? 1 : 0;
-  const int64_t e = dir ? s - a.n_edges : s;
-  const int32_t x = a.p1[e], y = a.p2[e];
-  src = dir ? y : x;
-  tgt = dir ? x : y;
-  const float st = a.rel_trans[src];
-  if (st == 0.0f) return false;                                        // :116
-  p = ((a.beta * a.layer_betas[e]) * st) * a.rel_sus[tgt];             // :117
-  if (p == 0.0f) return false;                                         // :118
-  double u;
-  if (a.uniforms) {
-    u = a.uniforms[dir * a.n_edges + e];
-  } else {
-    const uint64_t ue = (uint64_t)e;
-    const u32x4 w = philox_seeded(a.seed, (uint32_t)ue, (uint32_t)a.t,
-                                  STREAM_TX | ((uint32_t)a.variant << 8) | (uint32_t)a.layer, (uint32_t)(ue >> 32));
-    u = dir ? u01(w.z, w.w) : u01(w.x, w.y);
-  }
-  return u < (double)p;                                                // :123
+constexpr int INF_BLOCK = 1024;
+constexpr int INF_WAVES = INF_BLOCK / 64;
+constexpr int INF_CHUNK = 512;                 // edges: 8 per lane
+constexpr int INF_K = INF_CHUNK / 64;
+constexpr int INF_CHUNK_WORDS = INF_CHUNK / 32;
+constexpr int INF_WAVE_WORDS = INF_CHUNK / 2 + 2 * INF_CHUNK_WORDS;  // LDS: 16-bit queue of a chunk, its hit words
+constexpr int INF_MAX_GRID = 256;
+constexpr int64_t INF_CNT_WORDS = 2ll * INF_MAX_GRID * INF_WAVES;
+constexpr int INF_LDS = 0, INF_L2 = 1, INF_DIRECT = 2;
+
+__device__ inline uint32_t inf_lane() { return threadIdx.x & 63u; }
+__device__ inline uint32_t inf_below(uint64_t m) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+__device__ inline void inf_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+__device__ inline uint32_t inf_wave_sum(uint32_t v) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  return v;
 }
 
-constexpr int INF_BLOCK = 256;
-constexpr int INF_ITEMS = 8;
-constexpr int64_t INF_CHUNK = (int64_t)INF_BLOCK * INF_ITEMS;
-
-__global__ __launch_bounds__(INF_BLOCK) void infections_count_kernel(InfArgs a, uint32_t* __restrict__ block_counts) {
-  __shared__ uint32_t s_count;
-  if (threadIdx.x == 0) s_count = 0;
-  __syncthreads();
-  const int64_t base = (int64_t)blockIdx.x * INF_CHUNK;
-  uint32_t c = 0;
-  for (int j = 0; j < INF_ITEMS; ++j) {
-    const int64_t s = base + (int64_t)j * INF_BLOCK + threadIdx.x;
-    if (s < a.n_slots) {
-      int32_t src, tgt;
-      float p;
-      c += slot_transmits(a, s, src, tgt, p) ? 1u : 0u;
-    }
+__global__ __launch_bounds__(256) void infections_bits_kernel(InfArgs a) {
+  if (blockIdx.x == 0 && threadIdx.x < 2) a.out[threadIdx.x] = 0;
+  if (!a.bits) return;
+  const int64_t n_words = ((a.n_agents + 127) / 128) * 2;  // padded to 16 bytes
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n_words * 64; i += (int64_t)gridDim.x * 256) {
+    const uint64_t m = __ballot(i < a.n_agents && !(a.rel_trans[i] == 0.0f));  // :116
+    if (inf_lane() == 0) a.bits[i >> 6] = m;
   }
-  if (c) atomicAdd(&s_count, c);
-  __syncthreads();
-  if (threadIdx.x == 0) block_counts[blockIdx.x] = s_count;
 }
 
-// Exclusive scan of block counts in one workgroup (sequential chunks of 1024).
-__global__ __launch_bounds__(1024) void scan_counts_kernel(uint32_t* __restrict__ counts, int64_t n_blocks,
-                                                           uint64_t* __restrict__ total) {
-  __shared__ uint64_t s_vals[1024];
-  __shared__ uint64_t s_carry;
-  if (threadIdx.x == 0) s_carry = 0;
-  __syncthreads();
-  for (int64_t base = 0; base < n_blocks; base += 1024) {
-    const int64_t i = base + threadIdx.x;
-    const uint64_t v = i < n_blocks ? counts[i] : 0;
-    s_vals[threadIdx.x] = v;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-      const uint64_t add = threadIdx.x >= (unsigned)off ? s_vals[threadIdx.x - off] : 0;
-      __syncthreads();
-      s_vals[threadIdx.x] += add;
-      __syncthreads();
-    }
-    const uint64_t incl = s_vals[threadIdx.x];
-    if (i < n_blocks) counts[i] = (uint32_t)(s_carry + incl - v);  // offsets fit: capacity checked on host
-    __syncthreads();
-    if (threadIdx.x == 1023) s_carry += incl;
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) *total = s_carry;
+// This wave's chunks.
+__device__ inline void inf_range(const InfArgs& a, int64_t& c0, int64_t& c1) {
+  const int64_t w = (int64_t)blockIdx.x * INF_WAVES + (threadIdx.x >> 6), W = (int64_t)gridDim.x * INF_WAVES;
+  c0 = a.chunks * w / W;
+  c1 = a.chunks * (w + 1) / W;
 }
 
-__global__ __launch_bounds__(INF_BLOCK) void infections_write_kernel(InfArgs a, const uint32_t* __restrict__ offsets,
-                                                                     int64_t capacity, int32_t* __restrict__ src_out,
-                                                                     int32_t* __restrict__ tgt_out,
-                                                                     float* __restrict__ prob_out) {
-  __shared__ uint32_t s_scan[INF_BLOCK];
-  __shared__ uint32_t s_base;
-  if (threadIdx.x == 0) s_base = offsets[blockIdx.x];
-  __syncthreads();
-  const int64_t base = (int64_t)blockIdx.x * INF_CHUNK;
-  // Items are visited in slot order: round j covers slots base + j*BLOCK + [0, BLOCK).
-  for (int j = 0; j < INF_ITEMS; ++j) {
-    const int64_t s = base + (int64_t)j * INF_BLOCK + threadIdx.x;
-    int32_t src = 0, tgt = 0;
-    float p = 0.0f;
-    const bool hit = s < a.n_slots && slot_transmits(a, s, src, tgt, p);
-    s_scan[threadIdx.x] = hit ? 1u : 0u;
+template <int MODE>
+__global__ __launch_bounds__(INF_BLOCK) void infections_scan_kernel(InfArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint32_t s_inf[];
+  const uint32_t* map = s_inf;
+  if (MODE == INF_LDS) {
+    const uint4* src = (const uint4*)a.bits;
+    for (int j = threadIdx.x; j < (a.lds_words >> 2); j += INF_BLOCK) ((uint4*)s_inf)[j] = src[j];
     __syncthreads();
-    for (int off = 1; off < INF_BLOCK; off <<= 1) {
-      const uint32_t add = threadIdx.x >= (unsigned)off ? s_scan[threadIdx.x - off] : 0u;
-      __syncthreads();
-      s_scan[threadIdx.x] += add;
-      __syncthreads();
+  }
+  uint32_t* area = s_inf + (MODE == INF_LDS ? a.lds_words : 0) + (threadIdx.x >> 6) * INF_WAVE_WORDS;
+  uint16_t* queue = (uint16_t*)area;  // edge of the chunk | dir 0 << 9 | dir 1 << 10
+  uint32_t* s_hit = area + INF_CHUNK / 2;
+  const uint32_t lane = inf_lane();
+  const uint32_t n = (uint32_t)a.n_agents, nm1 = n ? n - 1u : 0u;
+  int64_t c0, c1;
+  inf_range(a, c0, c1);
+  uint32_t mine = 0, bad = 0;
+  for (int64_t c = c0; c < c1; ++c) {  // wave-uniform
+    const int64_t e0 = c * INF_CHUNK;
+    uint32_t x[INF_K], y[INF_K];
+#pragma unroll
+    for (int k = 0; k < INF_K; ++k) {
+      const int64_t e = e0 + k * 64 + lane;
+      x[k] = e < a.n_edges ? (uint32_t)a.p1[e] : 0u;
+      y[k] = e < a.n_edges ? (uint32_t)a.p2[e] : 0u;
     }
-    const uint32_t incl = s_scan[threadIdx.x];
-    const uint32_t round_total = s_scan[INF_BLOCK - 1];
-    if (hit) {
-      const int64_t pos = (int64_t)s_base + incl - 1;
-      if (pos < capacity) {
-        src_out[pos] = src;
-        tgt_out[pos] = tgt;
-        if (prob_out) prob_out[pos] = p;
+    uint32_t f1 = 0, f2 = 0;  // bit k: the direction's source can transmit
+#pragma unroll
+    for (int k = 0; k < INF_K; ++k) {
+      const bool in = e0 + k * 64 + lane < a.n_edges;
+      const bool ok = in && x[k] < n && y[k] < n;
+      bad |= in && !ok ? 1u : 0u;
+      const uint32_t xs = x[k] < nm1 ? x[k] : nm1, ys = y[k] < nm1 ? y[k] : nm1;
+      bool s1 = false, s2 = false;
+      if (ok) {
+        if (MODE == INF_DIRECT) {
+          s1 = !(a.rel_trans[xs] == 0.0f);
+          s2 = !(a.rel_trans[ys] == 0.0f);
+        } else {
+          const uint32_t* words = MODE == INF_LDS ? map : (const uint32_t*)a.bits;
+          s1 = (words[xs >> 5] >> (xs & 31u)) & 1u;
+          s2 = (words[ys >> 5] >> (ys & 31u)) & 1u;
+        }
+      }
+      f1 |= (uint32_t)s1 << k;
+      f2 |= (uint32_t)(s2 && a.dirs == 2) << k;
+    }
+    uint32_t n_q = 0;
+    inf_wave_sync();  // the previous chunk's words have been read
+#pragma unroll
+    for (int k = 0; k < INF_K; ++k) {
+      const bool cand = ((f1 | f2) >> k) & 1u;
+      const uint64_t m = __ballot(cand);
+      if (cand) queue[n_q + inf_below(m)] = (uint16_t)((k * 64 + lane) | (((f1 >> k) & 1u) << 9) | (((f2 >> k) & 1u) << 10));
+      n_q += (uint32_t)__popcll(m);
+    }
+    if (lane < 2 * INF_CHUNK_WORDS) s_hit[lane] = 0;
+    inf_wave_sync();
+    for (uint32_t r = 0; r < n_q; r += 64) {  // wave-uniform
+      if (r + lane < n_q) {
+        const uint32_t q = queue[r + lane], j = q & (INF_CHUNK - 1);
+        const int64_t e = e0 + j;
+        const int32_t xe = a.p1[e], ye = a.p2[e];
+        const float bl = a.beta * a.layer_betas[e];
+        float p[2] = {0.0f, 0.0f};
+        if (q & (1u << 9)) p[0] = (bl * a.rel_trans[xe]) * a.rel_sus[ye];   // :117
+        if (q & (1u << 10)) p[1] = (bl * a.rel_trans[ye]) * a.rel_sus[xe];
+        if (p[0] != 0.0f || p[1] != 0.0f) {                                 // :118
+          double u[2];
+          if (a.uniforms) {
+            u[0] = a.uniforms[e];
+            u[1] = p[1] != 0.0f ? a.uniforms[a.n_edges + e] : 1.0;
+          } else {
+            const uint64_t ue = (uint64_t)e;
+            const u32x4 w = philox_seeded(a.seed, (uint32_t)ue, (uint32_t)a.t,
+                                          STREAM_TX | ((uint32_t)a.variant << 8) | (uint32_t)a.layer, (uint32_t)(ue >> 32));
+            u[0] = u01(w.x, w.y);
+            u[1] = u01(w.z, w.w);
+          }
+#pragma unroll
+          for (int d = 0; d < 2; ++d)
+            if (p[d] != 0.0f && u[d] < (double)p[d])                        // :123
+              atomicOr(&s_hit[d * INF_CHUNK_WORDS + (j >> 5)], 1u << (j & 31u));
+        }
       }
     }
-    __syncthreads();
-    if (threadIdx.x == 0) s_base += round_total;
-    __syncthreads();
+    inf_wave_sync();
+    if (lane < (uint32_t)(a.dirs * INF_CHUNK_WORDS)) {
+      const uint32_t h = s_hit[lane];
+      a.hits[((int64_t)(lane / INF_CHUNK_WORDS) * a.chunks + c) * INF_CHUNK_WORDS + lane % INF_CHUNK_WORDS] = h;
+      mine += (uint32_t)__popc(h);
+    }
   }
+  const uint32_t n0 = inf_wave_sum(lane < INF_CHUNK_WORDS ? mine : 0u), n1 = inf_wave_sum(lane < INF_CHUNK_WORDS ? 0u : mine);
+  const int64_t w = (int64_t)blockIdx.x * INF_WAVES + (threadIdx.x >> 6);
+  if (lane == 0) {
+    a.cnt[w] = n0;
+    a.cnt[(int64_t)gridDim.x * INF_WAVES + w] = n1;
+  }
+  if (__ballot(bad != 0) && lane == 0) a.out[1] = 1;
+}
+
+// Same grid as the scan.
+__global__ __launch_bounds__(INF_BLOCK) void infections_write_kernel(InfArgs a, int64_t capacity, int32_t* src_out,
+                                                                     int32_t* tgt_out, float* prob_out) {
+  __shared__ unsigned long long s_sum[INF_WAVES][4];
+  const uint32_t lane = inf_lane(), wave = threadIdx.x >> 6;
+  const int W = (int)gridDim.x * INF_WAVES, first = (int)blockIdx.x * INF_WAVES;
+  // hits in all and before this workgroup, by direction
+  unsigned long long v[4] = {0, 0, 0, 0};
+  for (int j = threadIdx.x; j < W; j += INF_BLOCK) {
+    const uint32_t n0 = a.cnt[j], n1 = a.cnt[W + j];
+    v[0] += n0;
+    v[1] += n1;
+    v[2] += j < first ? n0 : 0u;
+    v[3] += j < first ? n1 : 0u;
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v[q] += __shfl_xor(v[q], off, 64);
+    if (lane == 0) s_sum[wave][q] = v[q];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    v[q] = 0;
+    for (int k = 0; k < INF_WAVES; ++k) v[q] += s_sum[k][q];
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) a.out[0] = v[0] + v[1];
+  int64_t c0, c1;
+  inf_range(a, c0, c1);
+  const unsigned long long start0 = v[2], start1 = v[0] + v[3];
+  for (int d = 0; d < a.dirs; ++d) {
+    uint64_t pos = d ? start1 : start0;
+    for (uint32_t k = 0; k < wave; ++k) pos += a.cnt[d * W + first + (int)k];
+    const uint32_t* hits = a.hits + (int64_t)d * a.chunks * INF_CHUNK_WORDS;
+    for (int64_t w0 = c0 * INF_CHUNK_WORDS; w0 < c1 * INF_CHUNK_WORDS; w0 += 64) {  // wave-uniform
+      uint32_t h = w0 + lane < c1 * INF_CHUNK_WORDS ? hits[w0 + lane] : 0u;
+      const uint32_t cnt = (uint32_t)__popc(h);
+      uint32_t incl = cnt;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t o = __shfl_up(incl, off, 64);
+        if ((int)lane >= off) incl += o;
+      }
+      int64_t at = (int64_t)(pos + incl - cnt);
+      while (h) {
+        const int64_t e = (w0 + lane) * 32 + (__ffs(h) - 1);
+        h &= h - 1;
+        const int32_t x = a.p1[e], y = a.p2[e];
+        const int32_t src = d ? y : x, tgt = d ? x : y;
+        if (at < capacity) {
+          src_out[at] = src;
+          tgt_out[at] = tgt;
+          if (prob_out) prob_out[at] = ((a.beta * a.layer_betas[e]) * a.rel_trans[src]) * a.rel_sus[tgt];
+        }
+        ++at;
+      }
+      pos += __shfl(incl, 63, 64);
+    }
+  }
+}
+
+static int64_t inf_chunks(int64_t n_edges) { return (n_edges + INF_CHUNK - 1) / INF_CHUNK; }
+static int64_t inf_bits_bytes(int64_t n_agents) { return ((n_agents + 127) / 128) * 16; }
+static int64_t inf_hits_bytes(int64_t n_edges) { return 2 * inf_chunks(n_edges) * INF_CHUNK_WORDS * 4; }
+
+// Where the scan finds the bitmap (see infections_scan_kernel) and its dynamic LDS. The limits are the device's.
+static int inf_lds_budget(int64_t* budget, int* n_cu) {
+  static thread_local int configured = -1;
+  static thread_local int64_t value = 0;
+  static thread_local int cus = 1;
+  int dev = -1;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0) return fail(CVK_E_HIP, "cvk_infections: no current device");
+  if (configured != dev) {
+    int lds = 0;
+    if (hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        hipFuncSetAttribute((const void*)infections_scan_kernel<INF_LDS>, hipFuncAttributeMaxDynamicSharedMemorySize, lds) !=
+            hipSuccess)
+      return fail(CVK_E_HIP, "cvk_infections: cannot query the device");
+    value = lds;
+    configured = dev;
+  }
+  *budget = value;
+  *n_cu = cus;
+  return CVK_OK;
 }
 
 }  // namespace cvk
@@ -244,30 +386,73 @@ static int infections_args(InfArgs& a, float beta, const int32_t* p1, const int3
   a.t = t;
   a.variant = variant;
   a.layer = layer;
-  a.n_slots = legacy ? n_edges : 2 * n_edges;
+  a.dirs = legacy ? 1 : 2;
+  a.n_agents = n_agents;
+  a.chunks = inf_chunks(n_edges);
   return CVK_OK;
 }
 
-// Count, scan, read the total back, write the ordered output. d_counts holds n_blocks block counts
-// (overwritten, so it need not start at zero), d_total one 64-bit word.
-static int infections_run(const InfArgs& a, int64_t n_blocks, uint32_t* d_counts, uint64_t* d_total,
-                          int32_t* src_out, int32_t* tgt_out, float* prob_out, int64_t capacity, int64_t* count_host,
-                          hipStream_t st, const char* name) {
-  hipLaunchKernelGGL(infections_count_kernel, dim3((unsigned)n_blocks), dim3(INF_BLOCK), 0, st, a, d_counts);
-  hipLaunchKernelGGL(scan_counts_kernel, dim3(1), dim3(1024), 0, st, d_counts, n_blocks, d_total);
-  uint64_t total = 0;
-  if (hipMemcpyAsync(&total, d_total, sizeof(uint64_t), hipMemcpyDeviceToHost, st) != hipSuccess ||
+// Runs the three launches; a's scratch pointers are set (a.bits may be null: rel_trans itself is gathered). Reads the
+// total back; *outside (if given) receives whether an endpoint lies outside [0, n_agents), an error otherwise.
+static int infections_run(InfArgs a, int32_t* src_out, int32_t* tgt_out, float* prob_out, int64_t capacity,
+                          int64_t* count_host, int32_t* outside, hipStream_t st, const char* name) {
+  int64_t budget = 0;
+  int n_cu = 1;
+  int rc = inf_lds_budget(&budget, &n_cu);
+  if (rc) return rc;
+  const int64_t queues = (int64_t)INF_WAVES * INF_WAVE_WORDS * 4, bits = inf_bits_bytes(a.n_agents);
+  const bool in_lds = a.bits && bits + queues <= budget;
+  a.lds_words = in_lds ? (int32_t)(bits / 4) : 0;
+  const int64_t bit_blocks = a.bits ? std::min<int64_t>((a.n_agents + 255) / 256, 2048) : 1;
+  hipLaunchKernelGGL(infections_bits_kernel, dim3((unsigned)std::max<int64_t>(bit_blocks, 1)), dim3(256), 0, st, a);
+  // a workgroup per CU (the bitmap takes most of its LDS), a chunk a wave at least
+  const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>(std::min(n_cu, INF_MAX_GRID), a.chunks));
+  const auto scan = !a.bits ? infections_scan_kernel<INF_DIRECT> : in_lds ? infections_scan_kernel<INF_LDS> : infections_scan_kernel<INF_L2>;
+  hipLaunchKernelGGL(scan, dim3(grid), dim3(INF_BLOCK), (size_t)((in_lds ? bits : 0) + queues), st, a);
+  hipLaunchKernelGGL(infections_write_kernel, dim3(grid), dim3(INF_BLOCK), 0, st, a, capacity, src_out, tgt_out, prob_out);
+  rc = check_launch(name);
+  if (rc) return rc;
+  uint64_t out[2] = {0, 0};
+  if (hipMemcpyAsync(out, a.out, sizeof(out), hipMemcpyDeviceToHost, st) != hipSuccess ||
       hipStreamSynchronize(st) != hipSuccess)
     return failf(CVK_E_HIP, "%s: count readback failed", name);
-  *count_host = (int64_t)total;
-  if ((int64_t)total > capacity) return failf(CVK_E_CAPACITY, "%s: output capacity too small", name);
-  if (total > 0)
-    hipLaunchKernelGGL(infections_write_kernel, dim3((unsigned)n_blocks), dim3(INF_BLOCK), 0, st, a, d_counts,
-                       capacity, src_out, tgt_out, prob_out);
-  const int rc = check_launch(name);
-  const hipError_t se = hipStreamSynchronize(st);
-  if (rc != CVK_OK) return rc;
-  return se == hipSuccess ? CVK_OK : failf(CVK_E_HIP, "%s: stream synchronize failed", name);
+  if (outside) *outside = out[1] ? 1 : 0;
+  if (out[1]) return outside ? CVK_OK : failf(CVK_E_INVALID, "%s: contact indices outside [0, n_agents)", name);
+  *count_host = (int64_t)out[0];
+  if ((int64_t)out[0] > capacity) return failf(CVK_E_CAPACITY, "%s: output capacity too small", name);
+  return CVK_OK;
+}
+
+// Scratch of one call, in a block of cvk_infections_work_bytes bytes (16-byte aligned).
+static void infections_scratch(InfArgs& a, char* base) {
+  a.out = (uint64_t*)base;
+  a.cnt = (uint32_t*)(base + 16);
+  a.bits = (uint64_t*)(base + 16 + INF_CNT_WORDS * 4);
+  a.hits = (uint32_t*)(base + 16 + INF_CNT_WORDS * 4 + inf_bits_bytes(a.n_agents));
+}
+
+extern "C" int64_t cvk_infections_work_bytes(int64_t n_edges, int64_t n_agents) {
+  if (n_edges < 0 || n_agents < 0) return 0;
+  return 16 + INF_CNT_WORDS * 4 + inf_bits_bytes(n_agents) + inf_hits_bytes(n_edges);
+}
+
+extern "C" int cvk_infections_work(float beta, const int32_t* p1, const int32_t* p2, const float* layer_betas,
+                                   int64_t n_edges, const float* rel_trans, const float* rel_sus, int64_t n_agents,
+                                   const double* uniforms, uint64_t seed, int32_t t, int32_t variant, int32_t layer,
+                                   int32_t legacy, int32_t* src_out, int32_t* tgt_out, float* prob_out,
+                                   int64_t capacity, int64_t* count_host, int32_t* outside_host, void* work,
+                                   int64_t work_bytes, void* stream) {
+  InfArgs a = {};
+  if (outside_host) *outside_host = 0;
+  const int rc = infections_args(a, beta, p1, p2, layer_betas, n_edges, rel_trans, rel_sus, n_agents, uniforms, seed, t,
+                                 variant, layer, legacy, src_out, tgt_out, capacity, count_host, "cvk_infections_work");
+  if (rc != CVK_OK) return rc == 1 ? CVK_OK : rc;
+  if (!work || ((uintptr_t)work & 15)) return fail(CVK_E_ALIGN, "cvk_infections_work: workspace must be 16-byte aligned");
+  if (work_bytes < cvk_infections_work_bytes(n_edges, n_agents))
+    return fail(CVK_E_CAPACITY, "cvk_infections_work: workspace too small");
+  infections_scratch(a, (char*)work);
+  return infections_run(a, src_out, tgt_out, prob_out, capacity, count_host, outside_host, (hipStream_t)stream,
+                        "cvk_infections_work");
 }
 
 extern "C" int cvk_infections(float beta, const int32_t* p1, const int32_t* p2, const float* layer_betas,
@@ -275,29 +460,26 @@ extern "C" int cvk_infections(float beta, const int32_t* p1, const int32_t* p2, 
                               const double* uniforms, uint64_t seed, int32_t t, int32_t variant, int32_t layer,
                               int32_t legacy, int32_t* src_out, int32_t* tgt_out, float* prob_out, int64_t capacity,
                               int64_t* count_host, void* stream) {
-  InfArgs a;
+  InfArgs a = {};
   int rc = infections_args(a, beta, p1, p2, layer_betas, n_edges, rel_trans, rel_sus, n_agents, uniforms, seed, t,
                            variant, layer, legacy, src_out, tgt_out, capacity, count_host, "cvk_infections");
   if (rc != CVK_OK) return rc == 1 ? CVK_OK : rc;
-  const int64_t n_blocks = (a.n_slots + INF_CHUNK - 1) / INF_CHUNK;
-  uint32_t* d_counts = nullptr;
-  if (hipMalloc((void**)&d_counts, (size_t)n_blocks * sizeof(uint32_t) + 64) != hipSuccess)
+  char* work = nullptr;
+  if (hipMalloc((void**)&work, (size_t)cvk_infections_work_bytes(n_edges, n_agents)) != hipSuccess)
     return fail(CVK_E_HIP, "cvk_infections: hipMalloc failed");
-  uint64_t* d_total = (uint64_t*)((char*)d_counts + ((n_blocks * sizeof(uint32_t) + 7) / 8) * 8);
-  rc = infections_run(a, n_blocks, d_counts, d_total, src_out, tgt_out, prob_out, capacity, count_host,
-                      (hipStream_t)stream, "cvk_infections");
-  (void)hipFree(d_counts);
+  infections_scratch(a, work);
+  rc = infections_run(a, src_out, tgt_out, prob_out, capacity, count_host, nullptr, (hipStream_t)stream, "cvk_infections");
+  (void)hipFree(work);
   return rc;
 }
 
 // ---- the same computation without allocation ----
-// Scratch of cvk_infections_noalloc: the per-block counts (CVK_INFECTIONS_NOALLOC_MAX_BLOCKS words),
-// then the 64-bit total. Every GPU the library runs on holds its own copy until the process ends.
-// In host code `scratch` only names the symbol; its device address comes from hipGetSymbolAddress,
-// once per device, and only that address is passed to kernels.
-static_assert(CVK_INFECTIONS_NOALLOC_MAX_SLOTS == CVK_INFECTIONS_NOALLOC_MAX_BLOCKS * INF_CHUNK,
-              "header limit and scratch size disagree");
-static __device__ __align__(256) uint32_t scratch[CVK_INFECTIONS_NOALLOC_MAX_BLOCKS + 64];
+// Scratch of cvk_infections_noalloc: the total, the waves' counts and the hit bits of the most slots it takes (16 MiB;
+// there is no room for a bit per agent of any population, so its scan gathers rel_trans itself). Every GPU the
+// library runs on holds its own copy until the process ends. In host code `scratch` only names the symbol; its device
+// address comes from hipGetSymbolAddress, once per device, and only that address is passed to kernels.
+constexpr int64_t NOALLOC_HIT_WORDS = CVK_INFECTIONS_NOALLOC_MAX_SLOTS / 32 + 2 * INF_CHUNK_WORDS;
+static __device__ __align__(256) uint32_t scratch[4 + INF_CNT_WORDS + NOALLOC_HIT_WORDS];
 
 namespace {
 constexpr int kMaxDevices = 64;
@@ -328,19 +510,21 @@ extern "C" int cvk_infections_noalloc(float beta, const int32_t* p1, const int32
                                       int32_t variant, int32_t layer, int32_t legacy, int32_t* src_out,
                                       int32_t* tgt_out, float* prob_out, int64_t capacity, int64_t* count_host,
                                       void* stream) {
-  InfArgs a;
+  InfArgs a = {};
   int rc = infections_args(a, beta, p1, p2, layer_betas, n_edges, rel_trans, rel_sus, n_agents, uniforms, seed, t,
                            variant, layer, legacy, src_out, tgt_out, capacity, count_host, "cvk_infections_noalloc");
   if (rc != CVK_OK) return rc == 1 ? CVK_OK : rc;
-  if (a.n_slots > CVK_INFECTIONS_NOALLOC_MAX_SLOTS)
+  const int64_t n_slots = a.dirs * n_edges;
+  if (n_slots > CVK_INFECTIONS_NOALLOC_MAX_SLOTS)
     return failf(CVK_E_CAPACITY, "cvk_infections_noalloc: %lld edge slots exceed the fixed scratch's limit of %lld "
                 "(use cvk_infections)",
-                (long long)a.n_slots, (long long)CVK_INFECTIONS_NOALLOC_MAX_SLOTS);
+                (long long)n_slots, (long long)CVK_INFECTIONS_NOALLOC_MAX_SLOTS);
   uint32_t* base = nullptr;
   rc = scratch_for_current_device(&base);
   if (rc != CVK_OK) return rc;
-  const int64_t n_blocks = (a.n_slots + INF_CHUNK - 1) / INF_CHUNK;
-  uint64_t* d_total = (uint64_t*)(base + CVK_INFECTIONS_NOALLOC_MAX_BLOCKS);  // 8-byte aligned: the block is a multiple of 64 words
-  return infections_run(a, n_blocks, base, d_total, src_out, tgt_out, prob_out, capacity, count_host,
-                        (hipStream_t)stream, "cvk_infections_noalloc");
+  a.out = (uint64_t*)base;
+  a.cnt = base + 4;
+  a.hits = base + 4 + INF_CNT_WORDS;
+  return infections_run(a, src_out, tgt_out, prob_out, capacity, count_host, nullptr, (hipStream_t)stream,
+                        "cvk_infections_noalloc");
 }

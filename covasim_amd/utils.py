@@ -77,7 +77,7 @@ def compute_trans_sus(rel_trans, rel_sus, inf, sus, beta_layer, viral_load, symp
     bools = []
     for name, b in [('inf', inf), ('sus', sus), ('symp', symp), ('iso', iso), ('quar', quar)]:
         bt, _ = _dev(b, np.bool_, name)
-        bools.append(bt.to(torch.uint8))
+        bools.append(bt.view(torch.uint8))
     n = rt.numel()
     for x in [rs, vl, imf] + bools:
         if x.numel() != n:
@@ -113,23 +113,29 @@ def compute_infections(beta, p1, p2, layer_betas, rel_trans, rel_sus, legacy=Fal
     n = rt.numel()
     if rs.numel() != n:
         raise ValueError('rel_trans and rel_sus must have equal lengths')
-    if E and (int(torch.minimum(a1.min(), a2.min())) < 0 or int(torch.maximum(a1.max(), a2.max())) >= n):
-        raise IndexError('contact indices outside [0, len(rel_trans))')
     u = None
     if uniforms is not None:
         u, _ = _dev(uniforms, np.float64, 'uniforms')
         if u.numel() != 2 * E:
+            if E and (int(torch.minimum(a1.min(), a2.min())) < 0 or int(torch.maximum(a1.max(), a2.max())) >= n):
+                raise IndexError('contact indices outside [0, len(rel_trans))')
             raise ValueError('uniforms must have shape (2, n_edges)')
     cap = (E if legacy else 2 * E)
     src = torch.empty(max(cap, 1), dtype=torch.int32, device=a1.device)
     tgt = torch.empty(max(cap, 1), dtype=torch.int32, device=a1.device)
-    prob = torch.empty(max(cap, 1), dtype=torch.float32, device=a1.device)
-    count = C.c_int64(0)
-    _lib.check(_lib.lib().cvk_infections(float(np.float32(beta)), _lib.ptr(a1), _lib.ptr(a2), _lib.ptr(lb), E,
-                                         _lib.ptr(rt), _lib.ptr(rs), n, _lib.ptr(u) if u is not None else None,
-                                         get_seed() & 0xFFFFFFFFFFFFFFFF, int(t), int(variant), int(layer),
-                                         1 if legacy else 0, _lib.ptr(src), _lib.ptr(tgt), _lib.ptr(prob), cap,
-                                         C.byref(count), _lib.stream_ptr()), 'compute_infections')
+    prob = torch.empty(max(cap, 1), dtype=torch.float32, device=a1.device) if return_probs else None
+    L = _lib.lib()
+    nbytes = int(L.cvk_infections_work_bytes(E, n))
+    work = torch.empty(nbytes, dtype=torch.uint8, device=a1.device)
+    count, outside = C.c_int64(0), C.c_int32(0)
+    _lib.check(L.cvk_infections_work(float(np.float32(beta)), _lib.ptr(a1), _lib.ptr(a2), _lib.ptr(lb), E, _lib.ptr(rt),
+                                     _lib.ptr(rs), n, _lib.ptr(u) if u is not None else None,
+                                     get_seed() & 0xFFFFFFFFFFFFFFFF, int(t), int(variant), int(layer),
+                                     1 if legacy else 0, _lib.ptr(src), _lib.ptr(tgt), _lib.ptr(prob), cap,
+                                     C.byref(count), C.byref(outside), _lib.ptr(work), nbytes, _lib.stream_ptr()),
+               'compute_infections')
+    if outside.value:
+        raise IndexError('contact indices outside [0, len(rel_trans))')
     k = count.value
     out = (_out(src[:k], is_t), _out(tgt[:k], is_t))
     if return_probs:

@@ -333,9 +333,19 @@ int cvk_infections(float beta, const int32_t* p1, const int32_t* p2, const float
                    int32_t legacy, int32_t* src_out, int32_t* tgt_out, float* prob_out, int64_t capacity,
                    int64_t* count_host, void* stream);
 
+/* The same in a workspace of the caller (device, 16-byte aligned, cvk_infections_work_bytes bytes). An endpoint
+ * outside [0, n_agents) is an error (CVK_E_INVALID) in all three; here, with outside_host given, it is reported there
+ * instead (1, and no pairs). */
+int64_t cvk_infections_work_bytes(int64_t n_edges, int64_t n_agents);
+int cvk_infections_work(float beta, const int32_t* p1, const int32_t* p2, const float* layer_betas,
+                        int64_t n_edges, const float* rel_trans, const float* rel_sus, int64_t n_agents,
+                        const double* uniforms, uint64_t seed, int32_t t, int32_t variant, int32_t layer,
+                        int32_t legacy, int32_t* src_out, int32_t* tgt_out, float* prob_out, int64_t capacity,
+                        int64_t* count_host, int32_t* outside_host, void* work, int64_t work_bytes, void* stream);
+
 /* No reference counterpart: cvk_infections without any allocation, for callers that cannot call
  * hipMalloc (serving loops, harnesses that forbid allocation). Same arguments, results and errors
- * as cvk_infections; its per-block counts live in a fixed device array of the library (256 KiB per
+ * as cvk_infections; its scratch is a fixed device array of the library (16 MiB per
  * GPU, held until the process ends) instead of a per-call allocation. Limit: at most
  * CVK_INFECTIONS_NOALLOC_MAX_SLOTS edge slots (2 * n_edges, or n_edges with legacy != 0); larger
  * calls return CVK_E_CAPACITY before any device work. Calls that overlap on one GPU (two host

@@ -119,6 +119,34 @@ def test_infections_philox_bit_exact(gpu):
         assert np.array_equal(s, ws) and np.array_equal(tg, wt)
 
 
+@pytest.mark.parametrize('legacy', [False, True])
+@pytest.mark.parametrize('n,E', [(1, 1), (64, 511), (65, 512), (129, 513), (3000, 70_001), (1_300_000, 200_003)])
+def test_infections_chunk_edges_match_oracle(gpu, n, E, legacy):
+    """Edge counts at and around the scan's chunks, populations around a word of its bitmap and past its LDS stage
+    (1.3M agents), no, some and all agents infectious; an endpoint outside the population raises."""
+    import torch
+    import covasim_amd as cv
+    rng = np.random.default_rng(E)
+    p1, p2 = rng.integers(0, n, E).astype(np.int32), rng.integers(0, n, E).astype(np.int32)
+    lb = rng.choice([1.0, 0.0, 2.5], E, p=[0.9, 0.05, 0.05]).astype(np.float32)
+    rs = np.where(rng.random(n) < 0.8, rng.random(n), 0).astype(np.float32)
+    cv.utils.set_seed(41)
+    for share in (0.0, 0.1, 1.0):
+        rt = np.where(rng.random(n) < share, 0.1 + rng.random(n) * 3, 0).astype(np.float32)
+        got = cv.utils.compute_infections(0.3, p1, p2, lb, rt, rs, legacy=legacy, t=3, variant=1, layer=2, return_probs=True)
+        want = co.compute_infections(0.3, p1, p2, lb, rt, rs, lambda d, idx: px.edge_uniforms(41, 3, 1, 2, idx, d),
+                                     legacy=legacy)
+        assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1]), share
+        assert np.array_equal(bits(got[2]), bits(want[2]))
+    for bad in (-1, n):
+        q = p1.copy()
+        q[E // 2] = bad
+        with pytest.raises(IndexError):
+            cv.utils.compute_infections(0.3, torch.from_numpy(q).cuda(), torch.from_numpy(p2).cuda(),
+                                        torch.from_numpy(lb).cuda(), torch.from_numpy(rt).cuda(),
+                                        torch.from_numpy(rs).cuda(), legacy=legacy)
+
+
 def run_pair(pop, n_days=40, seed=1, variants=(), use_graph=None, **pars):
     import covasim_amd as cv
     gpars = dict(pars)
