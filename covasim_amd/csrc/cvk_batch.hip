@@ -107,7 +107,7 @@ __global__ __launch_bounds__(AGENT_BLOCK) void batch_day_begin_kernel(BatchCommo
   S.partials_f = C.partials_f;
   S.part_stride = C.part_stride;
   S.part_col = blockIdx.x;
-  agent_block<APT, false>(C.P, C.params[s], S, a.t, a.prologue, a.transitions);
+  agent_block<APT, false>(C.P, C.params[s], S, a.t, a.prologue, a.transitions, true);
 }
 
 struct BatchReduce {
@@ -373,7 +373,7 @@ __global__ __launch_bounds__(INFECT_BLOCK) void batch_infect_kernel(BatchCommon 
           hosp_max = prm.n_beds_hosp >= 0 && (int64_t)row[CVK_R_MID_SEVERE] > prm.n_beds_hosp;
           icu_max = prm.n_beds_icu >= 0 && (int64_t)row[CVK_R_MID_CRITICAL] > prm.n_beds_icu;
         }
-        infect_stage(C.P, prm, stage, lanes_below(m), g, x, C.n_total, (uint32_t)s, hosp_max, icu_max);
+        infect_stage(C.P, prm, stage, lanes_below(m), g, x, C.n_total, (uint32_t)s, hosp_max, icu_max, t, true);
         if ((int32_t)l < C.n_layers && ia.log_capacity > 0) {  // the source is only for the log
           const SegView& L = ia.segs[s * C.n_layers + (int32_t)l];
           source = key_source(x.key, L.p1, L.p2, (ia.gen_mask >> l) & 1u, prm.seed, t,

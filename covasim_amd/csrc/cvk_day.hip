@@ -52,12 +52,19 @@ struct DayBeginArgs {
   int32_t n_resample;
   uint32_t agent_blocks;
   int32_t clock_slot;   // >= 0: the launch's start time goes to work.day_clock[clock_slot]
+  int32_t sev;          // store sev_imm (agent_block)
   ResampleLayer rs[CVK_MAX_LAYERS];
 };
 
+// Agents per thread of the agent pass: one up to AGENTS_ONE_MAX agents, where the chip has lanes for all of them and
+// a thread's second agent (with waning its powers, some 800 instructions) only lengthens the pass; two above, where
+// the second agent's loads hide the first's. Whole runs, two -> one: 20k agents x 60 days 3.13 -> 2.83 ms, 100k x 90
+// 4.81 -> 4.62 ms.
 constexpr int AGENTS_PER_THREAD = 2;
-static_assert(AGENT_BLOCK * AGENTS_PER_THREAD == 512, "one coarse-map word per agent-pass workgroup");
+constexpr int64_t AGENTS_ONE_MAX = (int64_t)1 << 18;
+static int agents_per_thread_for(int64_t n) { return n <= AGENTS_ONE_MAX ? 1 : AGENTS_PER_THREAD; }
 
+template <int APT>
 __global__ __launch_bounds__(AGENT_BLOCK) void day_begin_kernel(cvk_people P, cvk_params prm, cvk_work W,
                                                                 DayBeginArgs a) {
   // the day's start on the device's constant-rate wall clock (work.day_clock, optional)
@@ -76,11 +83,11 @@ __global__ __launch_bounds__(AGENT_BLOCK) void day_begin_kernel(cvk_people P, cv
   }
   AgentSpan S;
   S.g0 = 0;
-  S.li0 = (int64_t)blockIdx.x * (AGENT_BLOCK * AGENTS_PER_THREAD);
+  S.li0 = (int64_t)blockIdx.x * (AGENT_BLOCK * APT);
   S.n_local = P.n;
   S.n_stride = P.n;
   S.bitmap = (uint64_t*)W.bitmap;
-  S.coarse = W.coarse;  // one word per block: AGENT_BLOCK * AGENTS_PER_THREAD == 512
+  S.coarse = W.coarse;  // a word or half a word per block
   S.rec = W.rec;
   S.bound = W.bound;
   S.aux = (uint64_t*)W.aux;  // null unless the day's edge pass reads target bits
@@ -88,7 +95,7 @@ __global__ __launch_bounds__(AGENT_BLOCK) void day_begin_kernel(cvk_people P, cv
   S.partials_f = W.partials_f;
   S.part_stride = CVK_MAX_REDUCE_BLOCKS;
   S.part_col = blockIdx.x;
-  agent_block<AGENTS_PER_THREAD, true>(P, prm, S, a.t, a.prologue, a.transitions);
+  agent_block<APT, true>(P, prm, S, a.t, a.prologue, a.transitions, a.sev != 0);
 }
 
 // Writes the day rows from the summed partial rows of day_begin (block-wide).
@@ -437,6 +444,7 @@ struct InfectArgs {
   int32_t partial;    // 1: flow counts go to the infect partial rows (reduced later), 0: atomics on the row
   uint32_t infect_blocks;  // workgroups [0, infect_blocks) infect; the rest resample day rs_t
   int32_t words;           // touched words per wave and sweep (infect_words)
+  int32_t sev_stored;      // the agent pass stored the day's sev_imm
   int32_t rs_t;
   int32_t n_resample;
   ResampleLayer rs[CVK_MAX_LAYERS];
@@ -504,7 +512,7 @@ __global__ __launch_bounds__(INFECT_BLOCK) void infect_pass_kernel(cvk_people P,
       int32_t source = -1;
       const uint32_t l = key_layer(x.key);
       if (inf) {
-        infect_stage(P, prm, stage, lanes_below(m), i, x, P.n, 0u, hosp_max, icu_max);
+        infect_stage(P, prm, stage, lanes_below(m), i, x, P.n, 0u, hosp_max, icu_max, t, ia.sev_stored != 0);
         if ((int32_t)l < ia.n_layers)
           source = key_source(x.key, ia.p1[l], ia.p2[l], (ia.gen_mask >> l) & 1u, prm.seed, t, (uint32_t)P.n);
       }
@@ -608,7 +616,7 @@ static int validate(const cvk_people* P, const cvk_params* prm, const cvk_work* 
   if (!people_ok(P)) return fail(CVK_E_INVALID, "people struct has a null pointer or n <= 0");
   if (!prm || prm->n_agents != P->n) return fail(CVK_E_INVALID, "params.n_agents does not match people.n");
   if (P->n >= (1ll << 31) - 1) return fail(CVK_E_INVALID, "more than 2^31-2 agents");
-  if ((int64_t)grid_for(P->n, AGENT_BLOCK * AGENTS_PER_THREAD) > INFECT_PART_BASE)
+  if ((int64_t)grid_for(P->n, AGENT_BLOCK * agents_per_thread_for(P->n)) > INFECT_PART_BASE)
     return fail(CVK_E_CAPACITY, "too many agents for the reduction workspace (CVK_MAX_REDUCE_BLOCKS)");
   if (prm->n_variants < 1 || prm->n_variants > CVK_MAX_VARIANTS)
     return fail(CVK_E_INVALID, "n_variants must be in [1, 8]");
@@ -622,7 +630,7 @@ static int validate(const cvk_people* P, const cvk_params* prm, const cvk_work* 
   return CVK_OK;
 }
 
-static uint32_t agent_blocks_for(int64_t n) { return (uint32_t)grid_for(n, AGENT_BLOCK * AGENTS_PER_THREAD); }
+static uint32_t agent_blocks_for(int64_t n) { return (uint32_t)grid_for(n, AGENT_BLOCK * agents_per_thread_for(n)); }
 
 static int day_reduce_launch(cvk_work* work, const DayReduce& r, hipStream_t st) {
   if (!r.n_blocks && !r.infect_blocks) return CVK_OK;
@@ -662,12 +670,13 @@ static bool target_bits_for(int64_t n, const cvk_work* work);
 
 static int day_begin_launch(const cvk_people* people, const cvk_layer* layers, const cvk_params* params,
                             cvk_work* work, int32_t t, int prologue, int transitions, int resample, hipStream_t st,
-                            DayReduce* reduce_out) {
+                            DayReduce* reduce_out, bool sev = true) {
   DayBeginArgs a;
   memset(&a, 0, sizeof(a));
   a.t = t;
   a.prologue = prologue;
   a.transitions = transitions;
+  a.sev = sev ? 1 : 0;
   a.agent_blocks = agent_blocks_for(people->n);
   a.clock_slot = transitions ? t : t + 1;  // a closing pass marks the end of day t
   uint32_t rs_blocks = 0;
@@ -675,8 +684,8 @@ static int day_begin_launch(const cvk_people* people, const cvk_layer* layers, c
   if (rc) return rc;
   cvk_work w = *work;
   if (!(transitions && target_bits_for(people->n, work))) w.aux = nullptr;  // the target bits are for the edge pass
-  hipLaunchKernelGGL(day_begin_kernel, dim3(a.agent_blocks + rs_blocks), dim3(AGENT_BLOCK), 0, st, *people, *params,
-                     w, a);
+  hipLaunchKernelGGL(agents_per_thread_for(people->n) == 1 ? day_begin_kernel<1> : day_begin_kernel<AGENTS_PER_THREAD>,
+                     dim3(a.agent_blocks + rs_blocks), dim3(AGENT_BLOCK), 0, st, *people, *params, w, a);
   reduce_out->n_blocks = a.agent_blocks;
   reduce_out->t = t;
   reduce_out->prologue = prologue;
@@ -847,7 +856,8 @@ extern "C" int cvk_resample_layer(const cvk_layer* layer, int32_t layer_index, c
   cvk_work W;
   memset(&W, 0, sizeof(W));
   const int blocks = (int)std::min<int64_t>(grid_for(layer->n_edges, AGENT_BLOCK), 4 * std::max(caps().n_cu, 1));
-  hipLaunchKernelGGL(day_begin_kernel, dim3(blocks), dim3(AGENT_BLOCK), 0, (hipStream_t)stream, P, *params, W, a);
+  hipLaunchKernelGGL(day_begin_kernel<AGENTS_PER_THREAD>, dim3(blocks), dim3(AGENT_BLOCK), 0, (hipStream_t)stream, P,
+                     *params, W, a);
   return check_launch("cvk_resample_layer");
 }
 
@@ -1041,7 +1051,7 @@ extern "C" int cvk_edge_pass(const cvk_people* people, const cvk_layer* layers, 
 // the caller sets generate so that no source lookup reads a layer being rewritten.
 static int infect_impl(const cvk_people* people, const cvk_layer* layers, const cvk_params* params, cvk_work* work,
                        int32_t t, int32_t count_flows, int32_t allow_beds, hipStream_t st, bool generate = false,
-                       uint32_t* partial_blocks = nullptr, int32_t resample_t = -1) {
+                       uint32_t* partial_blocks = nullptr, int32_t resample_t = -1, bool sev_stored = true) {
   InfectArgs ia;
   memset(&ia, 0, sizeof(ia));
   for (int l = 0; l < params->n_layers; ++l) {
@@ -1053,6 +1063,7 @@ static int infect_impl(const cvk_people* people, const cvk_layer* layers, const 
   ia.n_layers = params->n_layers;
   ia.count_flows = count_flows;
   ia.allow_beds = allow_beds;
+  ia.sev_stored = sev_stored ? 1 : 0;
   const int grid = (int)infect_blocks_for(people->n, std::max(caps().n_cu, 1), INFECT_PART_BLOCKS);
   ia.words = infect_words((people->n + 31) / 32, (int64_t)grid * (INFECT_BLOCK / 64));
   ia.partial = partial_blocks && count_flows ? 1 : 0;
@@ -1139,7 +1150,9 @@ static int run_days_impl(const cvk_people* people, cvk_layer* layers, const cvk_
     DayReduce r;
     // the first resample of the run also sets every weight to 1; later ones leave them as they are
     const int rs_mode = gen ? 0 : (t == t0 ? 2 : (overlap ? 0 : 1));
-    rc = day_begin_launch(people, layers, params, work, t, t > t0 ? 1 : 0, 1, rs_mode, st, &r);
+    // sev_imm is stored on the run's last day only; the infect passes before it compute their targets' own
+    const bool sev = !params->use_waning || t + 1 == t1;
+    rc = day_begin_launch(people, layers, params, work, t, t > t0 ? 1 : 0, 1, rs_mode, st, &r, sev);
     if (rc) return rc;
     r.infect_blocks = infect_blocks;  // the previous day's flow counts
     r.infect_t = t - 1;
@@ -1160,7 +1173,7 @@ static int run_days_impl(const cvk_people* people, cvk_layer* layers, const cvk_
     if (rc) return rc;
     // tomorrow's resample (once today's edges have been read) with today's infections
     rc = infect_impl(people, layers, params, work, t, 1, 1, st, gen || overlap, &infect_blocks,
-                     overlap && t + 1 < t1 ? t + 1 : -1);
+                     overlap && t + 1 < t1 ? t + 1 : -1, sev);
     if (rc) return rc;
   }
   // close the last day: stocks and NAb update, and (generated layers) the last day's contacts, weights 1

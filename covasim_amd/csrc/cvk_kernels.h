@@ -230,7 +230,7 @@ struct AgentSpan {
   int64_t n_stride;    // row stride of the [variant][agent] arrays (all agents in storage)
   uint64_t* bitmap;    // the sim's infectious bitmap (64 agents per word, local indexing)
   uint32_t* coarse;    // one bit per 16 agents (OR of bitmap bits), one word per 512 agents; null: not
-                       // written (needs AGENT_BLOCK * APT == 512 and li0 a multiple of 512)
+                       // written (needs APT 1 or 2 and li0 a multiple of AGENT_BLOCK * APT)
   uint64_t* rec;       // the sim's edge records (local indexing)
   uint16_t* bound;     // the sim's upper-bound codes (local indexing)
   uint64_t* aux;       // the sim's target bits (susceptible with rel_sus != 0, not infectious) and, in the
@@ -246,9 +246,13 @@ struct AgentSpan {
 // stock counts of day tc = transitions ? t - 1 : t (sim.py:651-674). Block-wide.
 // LAZY: load the dates and factors in a second round trip, only where the state uses them (fewer
 // bytes on quiet days); otherwise every field is loaded in one round trip.
+// sev: compute and store sev_imm too. Else the day's infect pass computes it for its targets (infect_sev_imm); its
+// only other reader is the state after the run's last day. A third of the pass's powers, which bound it late in a run
+// with waning: 10M agents x 60 days 152.4 -> 150.3 ms. The batched pass always stores: there the powers hide behind
+// the loads, and its infect pass, with many more targets a day, took longer by them (95.3 -> 95.9 ms).
 template <int APT, bool LAZY>
 __device__ void agent_block(const cvk_people& P, const cvk_params& prm, const AgentSpan& S, int32_t t,
-                            int32_t prologue, int32_t transitions) {
+                            int32_t prologue, int32_t transitions, bool sev) {
   // per-wave counters: sums of per-agent booleans via ballot (wave-uniform, no shuffles)
   uint32_t c[N_AGENT_COLS];
 #pragma unroll
@@ -366,13 +370,13 @@ __device__ void agent_block(const cvk_people& P, const cvk_params& prm, const Ag
             if (eff != prev_eff) {  // variants with the same cross-immunity share the three powers
               ve_sus = calc_ve(eff, prm.ve_exp_alpha[0], prm.ve_beta[0]);
               ve_symp = calc_ve(eff, prm.ve_exp_alpha[1], prm.ve_beta[1]);
-              ve_sev = calc_ve(eff, prm.ve_exp_alpha[2], prm.ve_beta[2]);
+              if (sev) ve_sev = calc_ve(eff, prm.ve_exp_alpha[2], prm.ve_beta[2]);  // uniform
               prev_eff = eff;
             }
             const int64_t off = (int64_t)v * S.n_stride + g;
             P.sus_imm[off] = ve_sus;
             P.symp_imm[off] = ve_symp;
-            P.sev_imm[off] = ve_sev;
+            if (sev) P.sev_imm[off] = ve_sev;
           }
         }
         // viral-load phase (utils.py:58-78): early iff (t - start)/total < switch point
@@ -478,7 +482,8 @@ __device__ void agent_block(const cvk_people& P, const cvk_params& prm, const Ag
     uint32_t cw = 0;
 #pragma unroll
     for (int j = 0; j < AGENT_BLOCK / 64; ++j) cw |= s_coarse[j];
-    S.coarse[S.li0 >> 9] = cw;
+    if (APT == 1) ((uint16_t*)S.coarse)[S.li0 >> 8] = (uint16_t)cw;  // half a word per 256 agents
+    else S.coarse[S.li0 >> 9] = cw;
   }
 }
 
@@ -1244,14 +1249,25 @@ __device__ inline InfectIn infect_load(const cvk_people& P, const uint64_t* winn
 // The key names a susceptible target (people.py:470 keeps susceptibles only).
 __device__ inline bool infect_valid(const InfectIn& x) { return x.key != KEY_NONE && (x.f & CVK_SUSCEPTIBLE); }
 
+// sev_imm of the target for variant v as the day's agent pass would have stored it (check_immunity,
+// immunity.py:303-350, from the same state): agents without NAbs keep theirs.
+__device__ inline float infect_sev_imm(const cvk_params& prm, const InfectIn& x, uint32_t v, int32_t t) {
+  if (x.peak == 0.0f) return x.sev_imm;
+  const uint32_t rv = rec_var(x.vs);
+  const double imm = ((float)t >= x.drec && rv < MAXV) ? (double)prm.immunity[v][rv] : 0.0;
+  return calc_ve((double)x.nab * imm, prm.ve_exp_alpha[2], prm.ve_beta[2]);
+}
+
 // Entry j of the stage from a valid target's inputs. stride: row stride of the [variant][agent] arrays.
 __device__ inline void infect_stage(const cvk_people& P, const cvk_params& prm, InfectStage& S, uint32_t j, int64_t g,
-                                    InfectIn x, int64_t stride, uint32_t sim, bool hosp_max, bool icu_max) {
+                                    InfectIn x, int64_t stride, uint32_t sim, bool hosp_max, bool icu_max, int32_t t,
+                                    bool sev_stored) {
   const uint32_t v = key_variant(x.key);
   if (v) {
     x.symp_imm = gmem(P.symp_imm)[(int64_t)v * stride + g];
     x.sev_imm = gmem(P.sev_imm)[(int64_t)v * stride + g];
   }
+  if (!sev_stored && prm.use_waning) x.sev_imm = infect_sev_imm(prm, x, v, t);
   const bool new_peak = prm.use_waning && !(x.nab > 0.0f);
   S.g[j] = (int32_t)g;
   S.tag[j] = v | ((uint32_t)!isnan(x.drec) << 4) | ((uint32_t)new_peak << 5) | (sim << 8);

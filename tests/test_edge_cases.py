@@ -61,3 +61,22 @@ def test_infection_counts_per_wave_match_oracle(gpu, n, k):
     log = sim.infection_log()
     assert sorted(r['target'] for r in log) == sorted(tg for (_, tg, _, _, _) in osim.people.infection_log)
     assert len(log) == k and all(r['source'] is None and r['layer'] == 'seed_infection' for r in log)
+
+
+@pytest.mark.parametrize('n', [255, 257, 511, 513, 262_143, 262_145])
+def test_agent_pass_block_edges_match_oracle(gpu, n):
+    """One agent per thread up to 2^18 agents, two above, with the infectious map of 512-agent words (not the bitmap)
+    in LDS: half-written words, and reinfections on the days whose severity immunity is not stored."""
+    from covasim_amd import _lib
+    from tests.test_gpu_parity import assert_people_equal, assert_results_equal, run_pair
+    print(f'{n} agents', flush=True)
+    pop = make_population(n=n, pop_type='random')
+    days = 60 if n < 1000 else 5
+    _lib.check(_lib.lib().cvk_set_tuning(_lib.TUNE_EDGE_LDS, 0), 'tuning')
+    try:
+        sim, osim, ores = run_pair(copy_pop(pop), n_days=days, seed=3, pop_type='random', use_waning=True,
+                                   pop_infected=n // 8, beta=0.05)
+    finally:
+        _lib.check(_lib.lib().cvk_set_tuning(_lib.TUNE_EDGE_LDS, 1), 'tuning')
+    assert_results_equal(sim, ores)
+    assert_people_equal(sim, osim)
