@@ -1026,8 +1026,11 @@ static int edge_pass_impl(const cvk_people* people, const cvk_layer* layers, con
   a.agent_blocks = (uint32_t)agent_blocks_for(people->n);
   const int64_t work_items = std::max(wave_tiles, src_items);
   if (work_items == 0) return reduce ? day_reduce_launch(work, *reduce, st) : CVK_OK;
-  // one workgroup per CU (the LDS bitmap takes most of a CU's LDS), at least one work item each
-  const int grid = (int)std::min<int64_t>((work_items + EDGE_WAVES - 1) / EDGE_WAVES, (int64_t)std::max(c.n_cu, 1));
+  // One workgroup per CU (the LDS bitmap takes most of a CU's LDS), and one for the reduction. With fewer work items
+  // than the chip has waves they spread over all CUs, a few waves of a workgroup each: a wave's draws run alone on
+  // its SIMD instead of beside three others. 20k agents x 60 days 2.83 -> 2.75 ms, 100k x 90 4.62 -> 4.54 ms.
+  const int grid = (int)std::min<int64_t>(work_items + (a.reduce.n_blocks || a.reduce.infect_blocks ? 1 : 0),
+                                          (int64_t)std::max(c.n_cu, 1));
   const size_t shmem = (size_t)((int64_t)a.lds_words * 4 + queue_bytes);
   bool any_gen = false;
   for (int l = 0; l < params->n_layers; ++l) any_gen = any_gen || a.seg[l].gen;

@@ -68,43 +68,46 @@ __device__ inline float calc_ve(double nab, double exp_alpha, double beta) {
 // Reductions without device-scope fences: every block of a reducing kernel stores its partial
 // row (column-major, `stride` entries per column); the rows are summed after the kernel
 // boundary. Integer columns are order-free; float columns are summed in a fixed order.
-// Sums blocks [b0, b0 + nb) of every column (one wave per column, 8 loads in flight per lane);
+// Sums blocks [b0, b0 + nb) of every column (one wave per column, 4 columns of 8 loads in flight per lane);
 // totals land in s_tot[NC] / s_totf[ND]. Block-wide (contains a barrier).
 // ---------------------------------------------------------------------------
+template <class T, int NC, class Sum>
+__device__ inline void sum_columns(const T* partials, int64_t stride, uint32_t b0, uint32_t nb, T* s_tot, const Sum& wave_total) {
+  constexpr int COLS = 4;  // columns of a wave whose loads are in flight together
+  const int n_waves = (int)(blockDim.x >> 6);
+  for (int k0 = (int)(threadIdx.x >> 6); k0 < NC; k0 += COLS * n_waves) {
+    T acc[COLS][8];
+#pragma unroll
+    for (int q = 0; q < COLS; ++q)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) acc[q][j] = (T)0;
+    for (uint32_t c0 = 0; c0 < nb; c0 += 512) {
+#pragma unroll
+      for (int q = 0; q < COLS; ++q) {
+        if (k0 + q * n_waves >= NC) break;  // wave-uniform
+        const CVK_GLOBAL T* col = gmem(partials) + (size_t)(k0 + q * n_waves) * stride + b0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const uint32_t b = c0 + j * 64 + lane_id();
+          acc[q][j] += b < nb ? col[b] : (T)0;
+        }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < COLS; ++q) {
+      if (k0 + q * n_waves >= NC) break;
+      T tot = ((acc[q][0] + acc[q][1]) + (acc[q][2] + acc[q][3])) + ((acc[q][4] + acc[q][5]) + (acc[q][6] + acc[q][7]));
+      tot = wave_total(tot);
+      if (lane_id() == 0) s_tot[k0 + q * n_waves] = tot;
+    }
+  }
+}
+
 template <int NC, int ND>
 __device__ void sum_partials(const uint32_t* partials, const double* partials_f, int64_t stride, uint32_t b0,
                              uint32_t nb, uint32_t* s_tot, double* s_totf) {
-  const int n_waves = (int)(blockDim.x >> 6);
-  const int w = threadIdx.x >> 6;
-  for (int k = w; k < NC + ND; k += n_waves) {
-    if (k < NC) {
-      const uint32_t* col = partials + (size_t)k * stride + b0;
-      uint32_t acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-      for (uint32_t c0 = 0; c0 < nb; c0 += 512) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const uint32_t b = c0 + j * 64 + lane_id();
-          acc[j] += b < nb ? col[b] : 0u;
-        }
-      }
-      uint32_t tot = ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]));
-      tot = wave_sum(tot);
-      if (lane_id() == 0) s_tot[k] = tot;
-    } else {
-      const double* col = partials_f + (size_t)(k - NC) * stride + b0;
-      double acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-      for (uint32_t c0 = 0; c0 < nb; c0 += 512) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const uint32_t b = c0 + j * 64 + lane_id();
-          acc[j] += b < nb ? col[b] : 0.0;
-        }
-      }
-      double tot = ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]));
-      tot = wave_sum_d(tot);
-      if (lane_id() == 0) s_totf[k - NC] = tot;
-    }
-  }
+  sum_columns<uint32_t, NC>(partials, stride, b0, nb, s_tot, [](uint32_t v) { return wave_sum(v); });
+  if (ND) sum_columns<double, ND>(partials_f, stride, b0, nb, s_totf, [](double v) { return wave_sum_d(v); });
   __syncthreads();
 }
 
