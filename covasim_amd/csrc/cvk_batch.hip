@@ -469,49 +469,12 @@ __global__ __launch_bounds__(AGENT_BLOCK) void batch_choose_hist_kernel(BatchCom
 __global__ __launch_bounds__(64) void batch_choose_select_kernel(ChooseState cs, int32_t n_sims, int pass) {
   const int32_t s = blockIdx.x;
   if (s >= n_sims || cs.k[s] == 0 || cs.all[s]) return;
-  uint32_t* h = cs.hist + (int64_t)s * 256;
-  const uint32_t lane = lane_id();
-  uint32_t b[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) b[j] = h[lane * 4 + j];
-  const uint32_t lane_total = (b[0] + b[1]) + (b[2] + b[3]);
-  uint32_t incl = lane_total;  // inclusive scan over lanes
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const uint32_t y = __shfl_up(incl, off, 64);
-    if ((int)lane >= off) incl += y;
-  }
-  const uint32_t total = __shfl(incl, 63, 64);
-  uint32_t remain = cs.remain[s];
-  __syncthreads();
-#pragma unroll
-  for (int j = 0; j < 4; ++j) h[lane * 4 + j] = 0;
-  if (pass == 0 && remain >= total) {
-    if (lane == 0) {
-      cs.all[s] = 1;
-      if (remain > total) cs.shortfall[s] = 1;
-    }
-    return;
-  }
-  // the first bin whose cumulative count reaches `remain`
-  uint32_t before = incl - lane_total;
-  int digit = -1;
-  uint32_t cum_before_digit = 0;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    if (digit < 0 && before + b[j] >= remain) {
-      digit = (int)(lane * 4 + j);
-      cum_before_digit = before;
-    }
-    before += b[j];
-  }
-  const uint64_t found = __ballot(digit >= 0);
-  const int first = __ffsll((unsigned long long)found) - 1;
-  if ((int)lane == first) {
-    const int shift = 56 - 8 * pass;
-    cs.prefix[s] |= (uint64_t)digit << shift;
-    cs.remain[s] = remain - cum_before_digit;
-  }
+  const ChooseDigit d = choose_digit(cs.hist + (int64_t)s * 256, cs.prefix[s], cs.remain[s], pass);
+  if (lane_id() != 0) return;
+  cs.prefix[s] = d.prefix;
+  cs.remain[s] = d.remain;
+  cs.all[s] = d.state;
+  if (d.shortfall) cs.shortfall[s] = 1;
 }
 
 template <int APT>
@@ -523,7 +486,7 @@ __global__ __launch_bounds__(AGENT_BLOCK) void batch_choose_mark_kernel(BatchCom
   if (cs.k[s] == 0) return;
   const BatchSim& B = C.sims[s];
   const uint64_t seed = C.params[s].seed;
-  const uint64_t thr = cs.all[s] ? ~0ull : cs.prefix[s];
+  const uint64_t thr = cs.all[s] == CHOOSE_ALL ? ~0ull : cs.prefix[s];
   const int64_t li0 = (int64_t)(blockIdx.x - B.b_off) * (AGENT_BLOCK * APT);
   for (int r = 0; r < APT; ++r) {
     const int64_t li = li0 + (int64_t)r * AGENT_BLOCK + threadIdx.x;

@@ -168,42 +168,24 @@ __global__ __launch_bounds__(256) void choose_hist_kernel(cvk_people P, cvk_work
   if (s_hist[threadIdx.x]) atomicAdd(&W.select_hist[threadIdx.x], s_hist[threadIdx.x]);
 }
 
-__global__ void choose_select_kernel(cvk_work W, int pass) {
-  if (threadIdx.x != 0) return;
+__global__ __launch_bounds__(64) void choose_select_kernel(cvk_work W, int pass) {
   if (W.ctl[CVK_CTL_SEL_ALL]) return;
-  uint32_t remain = W.ctl[CVK_CTL_SEL_REMAIN];
-  if (pass == 0) {
-    uint64_t total = 0;
-    for (int dd = 0; dd < 256; ++dd) total += W.select_hist[dd];
-    if (remain >= total) {  // everyone eligible is chosen
-      W.ctl[CVK_CTL_SEL_ALL] = 1;
-      if (remain > total) W.ctl[CVK_CTL_SEL_SHORT] = 1;
-      for (int dd = 0; dd < 256; ++dd) W.select_hist[dd] = 0;
-      return;
-    }
-  }
-  uint64_t prefix = ((uint64_t)W.ctl[CVK_CTL_SEL_PREFIX + 1] << 32) | W.ctl[CVK_CTL_SEL_PREFIX];
-  const int shift = 56 - 8 * pass;
-  uint32_t cum = 0;
-  int digit = 255;
-  for (int dd = 0; dd < 256; ++dd) {
-    const uint32_t h = W.select_hist[dd];
-    if (cum + h >= remain) { digit = dd; break; }
-    cum += h;
-  }
-  remain -= cum;
-  prefix |= (uint64_t)digit << shift;
-  W.ctl[CVK_CTL_SEL_PREFIX] = (uint32_t)prefix;
-  W.ctl[CVK_CTL_SEL_PREFIX + 1] = (uint32_t)(prefix >> 32);
-  W.ctl[CVK_CTL_SEL_REMAIN] = remain;
-  for (int dd = 0; dd < 256; ++dd) W.select_hist[dd] = 0;
+  const uint64_t prefix = ((uint64_t)W.ctl[CVK_CTL_SEL_PREFIX + 1] << 32) | W.ctl[CVK_CTL_SEL_PREFIX];
+  const ChooseDigit d = choose_digit(W.select_hist, prefix, W.ctl[CVK_CTL_SEL_REMAIN], pass);
+  if (lane_id() != 0) return;
+  W.ctl[CVK_CTL_SEL_PREFIX] = (uint32_t)d.prefix;
+  W.ctl[CVK_CTL_SEL_PREFIX + 1] = (uint32_t)(d.prefix >> 32);
+  W.ctl[CVK_CTL_SEL_REMAIN] = d.remain;
+  W.ctl[CVK_CTL_SEL_ALL] = (uint32_t)d.state;
+  if (d.shortfall) W.ctl[CVK_CTL_SEL_SHORT] = 1;
 }
 
 __global__ __launch_bounds__(256) void choose_mark_kernel(cvk_people P, cvk_work W, uint64_t seed, int32_t t,
                                                           uint32_t stream_id, int32_t sus_only, uint32_t layer_code,
                                                           uint32_t variant) {
-  const uint64_t thr = W.ctl[CVK_CTL_SEL_ALL] ? ~0ull
-                                              : ((uint64_t)W.ctl[CVK_CTL_SEL_PREFIX + 1] << 32) | W.ctl[CVK_CTL_SEL_PREFIX];
+  const uint64_t thr = W.ctl[CVK_CTL_SEL_ALL] == (uint32_t)CHOOSE_ALL
+                           ? ~0ull
+                           : ((uint64_t)W.ctl[CVK_CTL_SEL_PREFIX + 1] << 32) | W.ctl[CVK_CTL_SEL_PREFIX];
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < P.n; i += (int64_t)gridDim.x * 256) {
     if (sus_only && !(P.flags[i] & CVK_SUSCEPTIBLE)) continue;
     const uint64_t key = selection_key(seed, t, stream_id, (uint32_t)i);

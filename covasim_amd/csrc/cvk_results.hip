@@ -16,11 +16,13 @@
 
 #include "cvk_device.h"
 #include "cvk_host.h"
+#include "cvk_kernels.h"
 
 namespace cvk {
 namespace {
 
 constexpr int FIN_BLOCK = 256;
+constexpr int FINALIZE_BLOCK = 1024;
 constexpr int64_t REFF_CHUNK = 16384;
 constexpr int PW_BLOCK = 128;  // numpy's pairwise-summation block
 
@@ -144,7 +146,20 @@ struct FinArgs {
   double* scratch;  // [S][2][npts]
 };
 
-__global__ __launch_bounds__(FIN_BLOCK) void finalize_kernel(FinArgs a) {
+// Inclusive sum over the wave's lanes. Of whole numbers below 2^53 (counts): exact in any order.
+__device__ inline double wave_scan(double v) {
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const double y = __shfl_up(v, off, 64);
+    if ((int)lane_id() >= off) v += y;
+  }
+  return v;
+}
+
+// One workgroup per sim; nothing here is large, so latency bounds it: every loop runs over the days with all lanes, the
+// running sums as wave scans. With one thread per series and one each for the doubling time and R_eff it took 104 us
+// at 61 days of 20k agents and 332 us at 121 days of 1M; now 10 and 19 us.
+__global__ __launch_bounds__(FINALIZE_BLOCK) void finalize_kernel(FinArgs a) {
   const int s = blockIdx.x;
   const int T = a.npts, nv = a.nv;
   const uint32_t* R = a.results + (int64_t)s * T * CVK_R_COLS;
@@ -156,46 +171,48 @@ __global__ __launch_bounds__(FIN_BLOCK) void finalize_kernel(FinArgs a) {
   const double pop = (double)(a.agent_off[s + 1] - a.agent_off[s]);
   const double pi = a.pop_infected[s];
 
-  // running sums and copies: flows, stocks, by-variant series
+  // running sums and copies: flows, stocks, by-variant series; a wave per series, a lane per day
   const int n_tasks = CVK_F_N_FLOWS + CVK_F_N_STOCKS + 6 * nv;
-  for (int task = threadIdx.x; task < n_tasks; task += FIN_BLOCK) {
+  const int lane = (int)lane_id();
+  for (int task = (int)(threadIdx.x >> 6); task < n_tasks; task += FINALIZE_BLOCK / 64) {
+    int col;
+    double *plain, *cum = nullptr;
+    bool seeded = false;
     if (task < CVK_F_N_FLOWS) {
-      const int f = task, col = flow_col(f);
-      double* nw = row(CVK_F_NEW + f);
-      double* cm = row(CVK_F_CUM + f);
-      double acc = 0.0;
-      for (int t = 0; t < T; ++t) {
-        const double v = col >= 0 ? (double)R[(int64_t)t * CVK_R_COLS + col] : 0.0;
-        nw[t] = v;
-        acc += v;
-        cm[t] = f == FLOW_INFECTIONS ? acc + pi : acc;
-      }
+      col = flow_col(task);
+      plain = row(CVK_F_NEW + task);
+      cum = row(CVK_F_CUM + task);
+      seeded = task == FLOW_INFECTIONS;
     } else if (task < CVK_F_N_FLOWS + CVK_F_N_STOCKS) {
-      const int k = task - CVK_F_N_FLOWS;
-      double* st = row(CVK_F_STOCK + k);
-      for (int t = 0; t < T; ++t) st[t] = (double)R[(int64_t)t * CVK_R_COLS + stock_col(k)];
+      col = stock_col(task - CVK_F_N_FLOWS);
+      plain = row(CVK_F_STOCK + task - CVK_F_N_FLOWS);
     } else {
       const int j = task - CVK_F_N_FLOWS - CVK_F_N_STOCKS, k = j / nv, v = j % nv;
-      const int col = CVK_R_BYVAR + k * CVK_MAX_VARIANTS + v;
-      double acc = 0.0;
-      for (int t = 0; t < T; ++t) {
-        const double x = (double)R[(int64_t)t * CVK_R_COLS + col];
-        if (k < 4) {
-          vrow(CVK_FV_NEW + k, v)[t] = x;
-          acc += x;
-          // sim.py:785-786 adds pop_infected to the whole (n_variants, npts) cumulative array
-          vrow(CVK_FV_CUM + k, v)[t] = k == 0 ? acc + pi : acc;
-        } else {
-          vrow(k == 4 ? CVK_FV_N_EXPOSED : CVK_FV_N_INFECTIOUS, v)[t] = x;
-        }
+      col = CVK_R_BYVAR + k * CVK_MAX_VARIANTS + v;
+      if (k < 4) {
+        plain = vrow(CVK_FV_NEW + k, v);
+        cum = vrow(CVK_FV_CUM + k, v);
+        seeded = k == 0;  // sim.py:785-786 adds pop_infected to the whole (n_variants, npts) cumulative array
+      } else {
+        plain = vrow(k == 4 ? CVK_FV_N_EXPOSED : CVK_FV_N_INFECTIOUS, v);
       }
+    }
+    double before = 0.0;  // the series' sum over the days before this chunk
+    for (int t0 = 0; t0 < T; t0 += 64) {
+      const int t = t0 + lane;
+      const double x = t < T && col >= 0 ? (double)R[(int64_t)t * CVK_R_COLS + col] : 0.0;
+      if (t < T) plain[t] = x;
+      if (!cum) continue;  // uniform over the wave
+      const double acc = before + wave_scan(x);
+      if (t < T) cum[t] = seeded ? acc + pi : acc;
+      before = __shfl(acc, 63, 64);
     }
   }
   __syncthreads();
 
   // derived states, one lane per day (compute_states)
   const double count_recov = a.use_waning ? 0.0 : 1.0;
-  for (int t = threadIdx.x; t < T; t += FIN_BLOCK) {
+  for (int t = threadIdx.x; t < T; t += FINALIZE_BLOCK) {
     const double cd = row(CVK_F_CUM + FLOW_DEATHS)[t], crec = row(CVK_F_CUM + FLOW_RECOVERIES)[t];
     const double ne = row(CVK_F_STOCK + STOCK_EXPOSED)[t], ni = row(CVK_F_STOCK + STOCK_INFECTIOUS)[t];
     const double nr = row(CVK_F_STOCK + STOCK_RECOVERED)[t];
@@ -228,11 +245,11 @@ __global__ __launch_bounds__(FIN_BLOCK) void finalize_kernel(FinArgs a) {
   }
   __syncthreads();
 
-  if (threadIdx.x == 0) {  // compute_doubling
+  {  // compute_doubling
     const double* cum = row(CVK_F_CUM + FLOW_INFECTIONS);
     double* dt = row(CVK_F_DOUBLING_TIME);
     const int w = a.window;
-    for (int t = 0; t < T; ++t) {
+    for (int t = threadIdx.x; t < T; t += FINALIZE_BLOCK) {
       double v = NAN;
       if (t >= w) {
         const double now = cum[t], prev = cum[t - w];
@@ -244,46 +261,67 @@ __global__ __launch_bounds__(FIN_BLOCK) void finalize_kernel(FinArgs a) {
       dt[t] = v;
     }
   }
-  if (threadIdx.x == 64) {  // compute_r_eff, method 'daily'
-    double so = 0.0, si = 0.0;
-    int64_t n = 0;
-    for (int64_t c = a.chunk_first[s]; c < a.chunk_first[s + 1]; ++c) {
+
+  // compute_r_eff, method 'daily': mean infectious period (wave 0: lane l takes parts l, l + 64, ..)
+  __shared__ double s_mean;
+  if (threadIdx.x < 64) {
+    double so = 0.0, si = 0.0, n = 0.0;
+    for (int64_t c = a.chunk_first[s] + lane; c < a.chunk_first[s + 1]; c += 64) {
       so += a.parts[c].outcome_sum;
       si += a.parts[c].inf_sum;
-      n += a.parts[c].count;
+      n += (double)a.parts[c].count;
     }
-    const double mean_inf = n > 0 ? so / (double)n - si / (double)n : 0.0;
-    double* raw = a.scratch + (int64_t)s * 2 * T;
-    double* tmp = raw + T;
+    so = wave_sum_d(so);
+    si = wave_sum_d(si);
+    n = wave_sum_d(n);
+    if (lane == 0) s_mean = n > 0 ? so / n - si / n : 0.0;
+  }
+  __syncthreads();
+  double* raw = a.scratch + (int64_t)s * 2 * T;
+  double* tmp = raw + T;
+  double* out = row(CVK_F_R_EFF);
+  {
+    const double mean_inf = s_mean;
     const double* nw = row(CVK_F_NEW + FLOW_INFECTIONS);
     const double* imp = row(CVK_F_N_IMPORTS);
     const double* ninf = row(CVK_F_STOCK + STOCK_INFECTIOUS);
-    for (int t = 0; t < T; ++t) raw[t] = mean_inf * (ninf[t] > 0 ? (nw[t] - imp[t]) / ninf[t] : 0.0);
-    double* out = row(CVK_F_R_EFF);
-    if (T >= 3) {
-      const int ip = a.initial_period[s];
-      auto at = [raw](int64_t i) { return raw[i]; };
-      for (int i = 0; i < ip; ++i) raw[i] = pairwise_sum(at, i, ip - i) / (double)(ip - i);
-      // repeated convolution with (0.25, 0.5, 0.25), zero beyond the ends (np.convolve 'same')
-      for (int t = 0; t < T; ++t) out[t] = raw[t];
-      for (int r = 0; r < a.smoothing; ++r) {
-        for (int t = 0; t < T; ++t) {
-          double acc;
-          if (t == 0) acc = out[0] * 0.5 + out[1] * 0.25;
-          else if (t == T - 1) acc = out[T - 2] * 0.25 + out[T - 1] * 0.5;
-          else acc = out[t - 1] * 0.25 + out[t] * 0.5 + out[t + 1] * 0.25;
-          tmp[t] = acc;
-        }
-        for (int t = 0; t < T; ++t) out[t] = tmp[t];
-      }
-      const int sm = std::min(a.smoothing, T);
-      for (int t = 0; t < sm; ++t) {
-        out[t] = raw[t];
-        out[T - 1 - t] = raw[T - 1 - t];
-      }
-    } else {
-      for (int t = 0; t < T; ++t) out[t] = raw[t];
+    for (int t = threadIdx.x; t < T; t += FINALIZE_BLOCK) {
+      raw[t] = mean_inf * (ninf[t] > 0 ? (nw[t] - imp[t]) / ninf[t] : 0.0);
+      if (T < 3) out[t] = raw[t];
     }
+  }
+  if (T < 3) return;
+  __syncthreads();
+  // the first days become the mean from their day to the end of the period (of the days as they were)
+  const int ip = a.initial_period[s];
+  auto at = [raw](int64_t i) { return raw[i]; };
+  for (int i = threadIdx.x; i < ip; i += FINALIZE_BLOCK) tmp[i] = pairwise_sum(at, i, ip - i) / (double)(ip - i);
+  __syncthreads();
+  for (int t = threadIdx.x; t < T; t += FINALIZE_BLOCK) {
+    if (t < ip) raw[t] = tmp[t];
+    out[t] = raw[t];
+  }
+  // repeated convolution with (0.25, 0.5, 0.25), zero beyond the ends (np.convolve 'same'), out and tmp in turn
+  const double* from = out;
+  double* to = tmp;
+  for (int r = 0; r < a.smoothing; ++r) {
+    __syncthreads();
+    for (int t = threadIdx.x; t < T; t += FINALIZE_BLOCK) {
+      double acc;
+      if (t == 0) acc = from[0] * 0.5 + from[1] * 0.25;
+      else if (t == T - 1) acc = from[T - 2] * 0.25 + from[T - 1] * 0.5;
+      else acc = from[t - 1] * 0.25 + from[t] * 0.5 + from[t + 1] * 0.25;
+      to[t] = acc;
+    }
+    double* swap = to;
+    to = const_cast<double*>(from);
+    from = swap;
+  }
+  // the days nearer than `smoothing` to either end keep their own value (also where the two ends overlap)
+  const int sm = std::min(a.smoothing, T);
+  for (int t = threadIdx.x; t < T; t += FINALIZE_BLOCK) {
+    if (t < sm || t >= T - sm) out[t] = raw[t];
+    else if (from != out) out[t] = from[t];
   }
 }
 
@@ -487,7 +525,7 @@ extern "C" int cvk_finalize(const cvk_finalize_desc* desc, const uint32_t* resul
   a.out = out;
   a.out_v = out_variant;
   a.scratch = w.scratch;
-  hipLaunchKernelGGL(finalize_kernel, dim3(S), dim3(FIN_BLOCK), 0, st, a);
+  hipLaunchKernelGGL(finalize_kernel, dim3(S), dim3(FINALIZE_BLOCK), 0, st, a);
   if ((rc = check_launch("cvk_finalize"))) return rc;
   if (hipStreamSynchronize(st) != hipSuccess) return fail(CVK_E_HIP, "cvk_finalize: device error");
   return CVK_OK;
