@@ -158,7 +158,7 @@ __device__ inline double wave_scan(double v) {
 
 // One workgroup per sim; nothing here is large, so latency bounds it: every loop runs over the days with all lanes, the
 // running sums as wave scans. With one thread per series and one each for the doubling time and R_eff it took 104 us
-// at 61 days of 20k agents and 332 us at 121 days of 1M; now 10 and 19 us.
+// at 61 days of 20k agents and 332 us at 181 days of 1M; now 10 and 19 us.
 __global__ __launch_bounds__(FINALIZE_BLOCK) void finalize_kernel(FinArgs a) {
   const int s = blockIdx.x;
   const int T = a.npts, nv = a.nv;

@@ -478,3 +478,25 @@ def test_trace_scan_finds_every_contact(n):
     row = sim._w['results'][0].cpu().numpy()
     assert row[_lib.R_COL['new_quarantined']] == np.count_nonzero(contact & ~is_case)
     assert row[_lib.R_COL['new_isolated']] == len(cases)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('extra', [0, 1, 3])
+def test_capacity_just_above_the_cases_traces_all(extra):
+    """A tracing capacity of the first day's cases, or a few more, traces them all: the selection's threshold is above
+    every key although many keys share its first byte."""
+    import covasim_amd as cv
+
+    def run(capacity):
+        sim = cv.Sim(pop_size=20000, pop_type='hybrid', n_days=3, rand_seed=2, pop_infected=8000,
+                     interventions=[cv.test_prob(symp_prob=1.0, asymp_prob=1.0, test_delay=0),
+                                    cv.contact_tracing(trace_probs=1.0, trace_time=0, capacity=capacity)])
+        sim.run()
+        return sim
+    free = run(None)
+    cases = int(free.results['new_diagnoses'].values.max())
+    print(f'{cases} cases', flush=True)
+    assert cases > 1000
+    capped = run(cases + extra)
+    for key in ('new_quarantined', 'n_quarantined', 'new_infections', 'new_diagnoses'):
+        assert np.array_equal(free.results[key].values, capped.results[key].values), key
