@@ -843,12 +843,19 @@ extern "C" int cvk_resample_layer(const cvk_layer* layer, int32_t layer_index, c
   return check_launch("cvk_resample_layer");
 }
 
-static int choose_impl(const cvk_people* people, const cvk_params* params, cvk_work* work, int32_t t,
-                       uint32_t stream_id, int64_t k, int32_t susceptible_only, int32_t layer_code, int32_t variant,
-                       hipStream_t st) {
+static int check_choose(const cvk_people* people, const cvk_params* params, int64_t k, int32_t layer_code,
+                        int32_t variant) {
   if (k < 0 || k > people->n) return fail(CVK_E_INVALID, "cvk_choose: k outside [0, n]");
   if (layer_code < 0 || layer_code > 15 || variant < 0 || variant >= params->n_variants)
     return fail(CVK_E_INVALID, "cvk_choose: bad layer code or variant");
+  return CVK_OK;
+}
+
+static int choose_impl(const cvk_people* people, const cvk_params* params, cvk_work* work, int32_t t,
+                       uint32_t stream_id, int64_t k, int32_t susceptible_only, int32_t layer_code, int32_t variant,
+                       hipStream_t st) {
+  const int rc = check_choose(people, params, k, layer_code, variant);
+  if (rc) return rc;
   if (k == 0) return CVK_OK;
   const int grid = (int)std::min<int64_t>(grid_for(people->n, 256), 8 * std::max(caps().n_cu, 1));
   hipLaunchKernelGGL(choose_init_kernel, dim3(1), dim3(256), 0, st, *work, (uint32_t)k);
@@ -1108,16 +1115,18 @@ extern "C" int cvk_day_plan(const cvk_layer* layers, const cvk_params* params, c
   return CVK_OK;
 }
 
+// Days [from, to) of a run of days [t0, t1). infect_blocks: infect partial rows not yet added to their day's row
+// (0 at the run's start, carried from part to part).
 static int run_days_impl(const cvk_people* people, cvk_layer* layers, const cvk_params* params, cvk_work* work,
-                         int32_t t0, int32_t t1, int64_t pop_infected, const cvk_imports* imports, hipStream_t st) {
+                         int32_t t0, int32_t t1, int64_t pop_infected, const cvk_imports* imports, hipStream_t st,
+                         int32_t from, int32_t to, uint32_t& infect_blocks) {
   int rc;
   const bool diag = imports && imports->diag;
   bool gen, overlap;
   day_plan(layers, params, imports, t1 - t0, &gen, &overlap);
-  uint32_t infect_blocks = 0;  // infect partial rows not yet added to their day's row
   const bool sched = imports && imports->n_beta_days > 0 && imports->beta_v_days && imports->beta_layer_days;
   cvk_params day_params = *params;
-  for (int32_t t = t0; t < t1; ++t) {
+  for (int32_t t = from; t < to; ++t) {
     if (sched) {  // this day's rates; kernel arguments are copied at launch (and into a captured graph)
       const int32_t row = std::min<int32_t>(t, imports->n_beta_days - 1);
       memcpy(day_params.beta_v, imports->beta_v_days + (int64_t)row * CVK_MAX_VARIANTS, sizeof(day_params.beta_v));
@@ -1161,6 +1170,7 @@ static int run_days_impl(const cvk_people* people, cvk_layer* layers, const cvk_
                      overlap && t + 1 < t1 ? t + 1 : -1, sev);
     if (rc) return rc;
   }
+  if (to < t1) return CVK_OK;
   // close the last day: stocks and NAb update, and (generated layers) the last day's contacts, weights 1
   DayReduce r;
   rc = day_begin_launch(people, layers, params, work, t1 - 1, 0, 0, gen ? 2 : 0, st, &r);
@@ -1179,11 +1189,67 @@ static int check_run_args(const cvk_people* people, cvk_layer* layers, const cvk
   return check_diag_schedule(people, layers, params, work, imports);
 }
 
-extern "C" int cvk_graph_create(const cvk_people* people, cvk_layer* layers, const cvk_params* params,
-                                cvk_work* work, int32_t t0, int32_t t1, int64_t pop_infected,
-                                const cvk_imports* imports, void* stream, void** graph_exec_out);
-extern "C" int cvk_graph_launch(void* graph_exec, void* stream);
-extern "C" int cvk_graph_destroy(void* graph_exec);
+// Captures days [from, to) of a run (run_days_impl) on st and instantiates them.
+static int capture_days(const cvk_people* people, cvk_layer* layers, const cvk_params* params, cvk_work* work,
+                        int32_t t0, int32_t t1, int64_t pop_infected, const cvk_imports* imports, hipStream_t st,
+                        int32_t from, int32_t to, uint32_t& infect_blocks, hipGraphExec_t* exec) {
+  if (hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal) != hipSuccess)
+    return fail(CVK_E_HIP, "cvk_graph_create: hipStreamBeginCapture failed");
+  const int rc = run_days_impl(people, layers, params, work, t0, t1, pop_infected, imports, st, from, to, infect_blocks);
+  hipGraph_t graph = nullptr;
+  const hipError_t ec = hipStreamEndCapture(st, &graph);
+  if (rc) {
+    if (graph) (void)hipGraphDestroy(graph);
+    return rc;
+  }
+  if (ec != hipSuccess || !graph) return fail(CVK_E_HIP, "cvk_graph_create: hipStreamEndCapture failed");
+  const hipError_t ei = hipGraphInstantiate(exec, graph, nullptr, nullptr, 0);
+  (void)hipGraphDestroy(graph);
+  return ei == hipSuccess ? CVK_OK : fail(CVK_E_HIP, "cvk_graph_create: hipGraphInstantiate failed");
+}
+
+// What capture needs besides check_run_args, before it starts: a stream, and the edge kernels' LDS limits (not a
+// stream operation).
+static int check_capture(void* stream) {
+  if (!stream) return fail(CVK_E_INVALID, "cvk_graph_create: graph capture needs a non-default stream");
+  int64_t budget = 0;
+  return edge_dynamic_lds(&budget);
+}
+
+// Days of the first graph of a run, and the most of a later one (each has twice its predecessor's). One graph of all
+// days keeps the device idle while the host captures and instantiates it, some 45 us a day with testing and tracing,
+// half of what the device then takes: 121 days of 300k agents 16.0 ms as one graph, 12.0 ms in parts, of which only
+// the first is waited for.
+constexpr int32_t GRAPH_DAYS_FIRST = 4, GRAPH_DAYS_MAX = 32;
+
+static int run_days_graphs(const cvk_people* people, cvk_layer* layers, const cvk_params* params, cvk_work* work,
+                           int32_t t0, int32_t t1, int64_t pop_infected, const cvk_imports* imports, hipStream_t st) {
+  // an import event that choose_impl would refuse is refused before any day has run
+  for (int j = 0; imports && j < imports->n; ++j) {
+    if (imports->days[j] < t0 || imports->days[j] >= t1) continue;
+    const int rc = check_choose(people, params, imports->n_imports[j], CVK_LAYER_IMPORT, imports->variants[j]);
+    if (rc) return rc;
+  }
+  hipGraphExec_t parts[64];  // launched, not yet released
+  int n_parts = 0, rc = CVK_OK;
+  uint32_t infect_blocks = 0;
+  int32_t days = GRAPH_DAYS_FIRST;
+  for (int32_t from = t0; from < t1 && !rc; from += days, days = std::min(2 * days, GRAPH_DAYS_MAX)) {
+    const int32_t to = t1 - from <= days ? t1 : from + days;
+    hipGraphExec_t exec = nullptr;
+    rc = capture_days(people, layers, params, work, t0, t1, pop_infected, imports, st, from, to, infect_blocks, &exec);
+    if (rc) break;
+    parts[n_parts++] = exec;
+    if (hipGraphLaunch(exec, st) != hipSuccess) rc = fail(CVK_E_HIP, "cvk_run_days: hipGraphLaunch failed");
+    if (n_parts == 64) {  // some 2000 days: release what has run
+      (void)hipStreamSynchronize(st);
+      while (n_parts) (void)hipGraphExecDestroy(parts[--n_parts]);
+    }
+  }
+  (void)hipStreamSynchronize(st);
+  while (n_parts) (void)hipGraphExecDestroy(parts[--n_parts]);
+  return rc;
+}
 
 extern "C" int cvk_run_days(const cvk_people* people, cvk_layer* layers, const cvk_params* params, cvk_work* work,
                             int32_t t0, int32_t t1, int64_t pop_infected, const cvk_imports* imports,
@@ -1192,14 +1258,12 @@ extern "C" int cvk_run_days(const cvk_people* people, cvk_layer* layers, const c
   if (rc) return rc;
   if (t1 == t0) return CVK_OK;
   hipStream_t st = (hipStream_t)stream;
-  if (!use_graph) return run_days_impl(people, layers, params, work, t0, t1, pop_infected, imports, st);
-  void* exec = nullptr;
-  rc = cvk_graph_create(people, layers, params, work, t0, t1, pop_infected, imports, stream, &exec);
-  if (rc) return rc;
-  rc = cvk_graph_launch(exec, stream);
-  (void)hipStreamSynchronize(st);
-  (void)cvk_graph_destroy(exec);
-  return rc;
+  if (use_graph) {
+    rc = check_capture(stream);
+    return rc ? rc : run_days_graphs(people, layers, params, work, t0, t1, pop_infected, imports, st);
+  }
+  uint32_t infect_blocks = 0;
+  return run_days_impl(people, layers, params, work, t0, t1, pop_infected, imports, st, t0, t1, infect_blocks);
 }
 
 // Two-phase graph API: capture days [t0, t1) once, replay many times (inputs must be reset
@@ -1212,25 +1276,13 @@ extern "C" int cvk_graph_create(const cvk_people* people, cvk_layer* layers, con
   int rc = check_run_args(people, layers, params, work, t0, t1, imports);
   if (rc) return rc;
   if (t1 <= t0) return fail(CVK_E_INVALID, "cvk_graph_create: empty day range");
-  hipStream_t st = (hipStream_t)stream;
-  if (st == nullptr) return fail(CVK_E_INVALID, "cvk_graph_create: graph capture needs a non-default stream");
-  int64_t budget = 0;
-  rc = edge_dynamic_lds(&budget);  // not a stream operation: done before capture
+  rc = check_capture(stream);
   if (rc) return rc;
-  if (hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal) != hipSuccess)
-    return fail(CVK_E_HIP, "cvk_graph_create: hipStreamBeginCapture failed");
-  rc = run_days_impl(people, layers, params, work, t0, t1, pop_infected, imports, st);
-  hipGraph_t graph = nullptr;
-  const hipError_t ec = hipStreamEndCapture(st, &graph);
-  if (rc) {
-    if (graph) (void)hipGraphDestroy(graph);
-    return rc;
-  }
-  if (ec != hipSuccess || !graph) return fail(CVK_E_HIP, "cvk_graph_create: hipStreamEndCapture failed");
+  uint32_t infect_blocks = 0;
   hipGraphExec_t exec = nullptr;
-  const hipError_t ei = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-  (void)hipGraphDestroy(graph);
-  if (ei != hipSuccess) return fail(CVK_E_HIP, "cvk_graph_create: hipGraphInstantiate failed");
+  rc = capture_days(people, layers, params, work, t0, t1, pop_infected, imports, (hipStream_t)stream, t0, t1,
+                    infect_blocks, &exec);
+  if (rc) return rc;
   *graph_exec_out = (void*)exec;
   return CVK_OK;
 }

@@ -519,7 +519,8 @@ typedef struct {
 int cvk_day_plan(const cvk_layer* layers, const cvk_params* params, const cvk_imports* imports, int32_t n_days,
                  int32_t* out);
 /* Runs days [t0, t1) (t0 == 0 also seeds pop_infected infections first). use_graph != 0
- * captures the launches into one hipGraph and launches it once. */
+ * captures the launches into hipGraphs of a few days each, launches each one once as soon as it is there, and waits
+ * for the stream. */
 int cvk_run_days(const cvk_people* people, cvk_layer* layers, const cvk_params* params, cvk_work* work,
                  int32_t t0, int32_t t1, int64_t pop_infected, const cvk_imports* imports,
                  int32_t use_graph, void* stream);

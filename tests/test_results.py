@@ -211,3 +211,56 @@ def test_device_reduce_matches_numpy(S):
             want = rr.reduce(vals, quantiles=q, use_mean=kw.get('use_mean', False), bounds=kw.get('bounds', 2))
         for g, w in zip(got, want):
             assert np.array_equal(g, w, equal_nan=True), (kw, np.argwhere(~((g == w) | (np.isnan(g) & np.isnan(w))))[:5])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('days', [0, 1, 2, 3, 4, 11, 12, 27, 28, 59, 63, 64, 128])
+def test_day_counts_around_waves_and_graph_parts(days):
+    """Rows of days + 1 points against the restatement (the series are summed by waves of 64 days), from a run in
+    graphs of 4, 8, 16, 32, .. days on a stream of its own, which an eager run equals."""
+    import covasim_amd as cv
+    import torch
+    print(f'{days} days', flush=True)
+
+    def run(graph):
+        sim = cv.Sim(pop_size=3000, pop_type='hybrid', n_days=days, rand_seed=4, beta=0.03, use_waning=True,
+                     dynam_layer=dict(c=1), variants=[cv.variant(dict(rel_beta=1.5), days=2, n_imports=20)],
+                     interventions=[cv.test_prob(symp_prob=0.2, asymp_prob=0.01), cv.contact_tracing(trace_time=1)])
+        stream = torch.cuda.Stream() if graph else torch.cuda.current_stream()
+        with torch.cuda.stream(stream):
+            sim.run(use_graph=graph)
+        return sim
+    parts, eager = run(True), run(False)
+    for key, res in eager.results.items():
+        if hasattr(res, 'values') and not callable(res.values):
+            assert np.array_equal(res.values, parts.results[key].values, equal_nan=True), key
+    want, cvres = oracle_rows(parts)
+    assert_rows_match(parts, want, cvres)
+
+
+@pytest.mark.gpu
+def test_import_refused_before_a_graph_run_starts():
+    """An import event that cannot be drawn (a variant the run does not have) is refused before any day has run, also
+    where its day lies in a later graph than the first."""
+    import ctypes as C
+
+    import covasim_amd as cv
+    import torch
+    from covasim_amd import _lib
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        sim = cv.Sim(pop_size=2000, n_days=40, rand_seed=4,
+                     variants=[cv.variant(dict(rel_beta=1.5), days=30, n_imports=5)])
+        sim.initialize()
+        torch.cuda.synchronize()
+        imp = _lib.ImportsS.from_buffer_copy(sim._imports)
+        assert imp.n == 1
+        vars_ = (C.c_int32 * 1)(7)
+        imp.variants = C.cast(vars_, C.POINTER(C.c_int32))
+        before = sim.people.snapshot()
+        rc = _lib.lib().cvk_run_days(sim.people.struct(), sim._layers, sim._params, sim._work, 0, sim.npts, 20,
+                                     C.byref(imp), 1, C.c_void_p(stream.cuda_stream))
+        torch.cuda.synchronize()
+    assert rc != 0
+    after = sim.people.snapshot()
+    assert all(np.array_equal(before[k], after[k], equal_nan=True) for k in before)
