@@ -413,23 +413,16 @@ def run_relax(w, args):
     obs_t = torch.as_tensor(observed[:r32.n_days])
     loss_truth = float(log_incidence_loss(torch.as_tensor(r32.forward_np(theta)), obs_t))
     n, T = w['pop_size'], r32.n_days
-    # algorithmic HBM bytes of one forward + adjoint (every kernel; the neighbour gathers of tr, lbar and
-    # age bin are served from the caches and not counted): per day t a forward (relax_trans_kernel: rel_trans,
-    # bin, tr and min(t, kmax) past deltas; relax_forward_kernel: indptr (int64) per layer, bin, s read and
-    # written, delta, 4 per neighbour slot), the adjoint's recomputed forward (plus L and s recorded), and
-    # the adjoint (relax_adj_agent_kernel: bin, L, s, sbar r/w, lbar, min(kmax, T-1-t) ibar rows;
-    # relax_pack_kernel: tr, lbar, bin, the 16-byte neighbour record written; relax_adj_edge_kernel:
-    # indptr per layer, bin, tr, lbar, rel_trans, ibar written, 4 per slot)
+    # algorithmic HBM bytes of one forward + adjoint (the neighbour gathers are served from the caches and not
+    # counted): per day t a forward (relax_day_kernel: bin, rel_trans, s read and written, the end of the agent's
+    # list, delta, tr and the day's three records written, min(t, kmax) past deltas, 4 per neighbour slot) and the
+    # adjoint (relax_adjoint_kernel: bin, rel_trans, the list's end, the three records, tr of two days, lbar and
+    # sbar read and written, ibar written, min(kmax, T-1-t) ibar rows, 4 per slot)
     slots = int(sum(lay[1].numel() for lay in r32._csr if lay is not None))
-    n_dyn = sum(1 for c_l in r32.dyn_slots if c_l)
-    L_ = r32.n_layers
     kmax = min(r32.w.shape[1] - 1, T)
-    L_ = L_ - n_dyn  # the resampled layers have no lists: their expected term reads tr once (4 B per agent)
-    fwd = sum(n * (9 + 4 * min(t, kmax)) + n * (8 * L_ + 13) + 4 * n * (n_dyn > 0) + 4 * slots for t in range(T))
-    rec = 8 * n * T
-    adj = sum(n * (21 + 4 * min(kmax, T - 1 - t)) + n * 25 + n * (8 * L_ + 17) + 9 * n * (n_dyn > 0) + 4 * slots
-              for t in range(T))
-    fb_bytes = 2 * fwd + rec + adj
+    fwd = sum(n * (37 + 4 * min(t, kmax)) + 4 * slots for t in range(T))
+    adj = sum(n * (49 + 4 * min(kmax, T - 1 - t)) + 4 * slots for t in range(T))
+    fb_bytes = fwd + adj
     fb_gbs = fb_bytes / fb_ev_s / 1e9
     out = {
         'metric': METRIC, 'value': n * T / fb_s, 'unit': 'agent-days/s', 'n_gpus': 1, 'steps': T, 'warmup': 2 * T,
@@ -440,9 +433,8 @@ def run_relax(w, args):
         'roofline': {'bound': 'hbm', 'kernel': 'relaxation forward + adjoint (every kernel, 60 days)',
                      'achieved': fb_gbs, 'peak': HBM_PEAK_GBS, 'unit': 'GB/s', 'frac': fb_gbs / HBM_PEAK_GBS,
                      'traffic': None, 'algorithmic_bytes_per_step': fb_bytes, 'step_ms_hip_events': fb_ev_s * 1e3,
-                     'neighbour_slots': slots, 'note': 'the neighbour gathers (one 16-byte record per slot in the '
-                     'adjoint, one tr value in the forward) are served from L2 / MALL and bound the two edge '
-                     'kernels; they are not in the bytes'},
+                     'neighbour_slots': slots, 'note': 'the neighbour gathers (one value per slot) are served from L2 / MALL '
+                     'and bound both kernels; they are not in the bytes'},
         'relaxation': {'forward_ms': fwd_s * 1e3, 'forward_adjoint_ms': fb_s * 1e3,
                        'grad_rel_err_vs_fp64_central_fd': grad_err, 'fd_step_relative': h,
                        'calibration_iters': len(hist), 'calibration_s': cal_s,

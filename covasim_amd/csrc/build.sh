@@ -11,7 +11,7 @@ flags=(--offload-arch=gfx950 -O3 -std=c++17 -fPIC
        -ffp-contract=off -fhip-fp32-correctly-rounded-divide-sqrt -fno-gpu-rdc
        -Xclang -target-feature -Xclang -packed-fp32-ops
        -Wall -Wno-unused-function -DCVK_SOURCE_HASH="${src_hash}")
-# Loop-invariant code motion on machine code is off for the day loops: it lifts the constants of the infect
+# Loop-invariant code motion on machine code is off for the day loops and the relaxation: it lifts the constants of the infect
 # kernels' double-precision polynomials out of their round loop into registers (172 vector registers against 90,
 # and spills under a bound), and the edge kernels lose 5 to 14 registers to the same.
 day_flags=(-mllvm -disable-machine-licm)

@@ -11,8 +11,8 @@ a differentiable torch function of theta = [beta, beta_layer for each layer, rel
 the 10 prognosis age bins]. The model and its adjoint are spelled out in
 ``csrc/cvk_relax.hip``. The forward runs in float32 (precision=32, log-space products
 accumulated in float32) or float64 (precision=64). The gradient comes from the
-hand-written adjoint kernels, with the state checkpointed every ``checkpoint_every``
-days. ``calibrate`` fits theta to an observed daily-incidence curve with Adam on log(theta).
+hand-written adjoint kernels; every day's record is kept where half of the free memory
+takes them, else the state is checkpointed every ``checkpoint_every`` days. ``calibrate`` fits theta to an observed daily-incidence curve with Adam on log(theta).
 
 The per-agent relative transmissibility over time since infection,
 w_b(d) = E[infectious on lag d x viral load x asymptomatic factor], is tabulated per age
