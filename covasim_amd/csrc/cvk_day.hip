@@ -59,7 +59,8 @@ struct DayBeginArgs {
 // Agents per thread of the agent pass: one up to AGENTS_ONE_MAX agents, where the chip has lanes for all of them and
 // a thread's second agent (with waning its powers, some 800 instructions) only lengthens the pass; two above, where
 // the second agent's loads hide the first's. Whole runs, two -> one: 20k agents x 60 days 3.13 -> 2.83 ms, 100k x 90
-// 4.81 -> 4.62 ms.
+// 4.81 -> 4.62 ms, 280k x 60 equal; above, the twice as many partial rows cost the reduction more than that gains:
+// static layers x 60 days, two -> one, 500k 3.62 -> 3.83, 1M 4.14 -> 4.51, 3M 7.98 -> 9.1 ms.
 constexpr int AGENTS_PER_THREAD = 2;
 constexpr int64_t AGENTS_ONE_MAX = (int64_t)1 << 18;
 static int agents_per_thread_for(int64_t n) { return n <= AGENTS_ONE_MAX ? 1 : AGENTS_PER_THREAD; }
