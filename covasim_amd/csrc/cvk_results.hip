@@ -17,6 +17,7 @@
 #include "cvk_device.h"
 #include "cvk_host.h"
 #include "cvk_kernels.h"
+#include "cvk_smooth.h"
 
 namespace cvk {
 namespace {
@@ -297,32 +298,8 @@ __global__ __launch_bounds__(FINALIZE_BLOCK) void finalize_kernel(FinArgs a) {
   auto at = [raw](int64_t i) { return raw[i]; };
   for (int i = threadIdx.x; i < ip; i += FINALIZE_BLOCK) tmp[i] = pairwise_sum(at, i, ip - i) / (double)(ip - i);
   __syncthreads();
-  for (int t = threadIdx.x; t < T; t += FINALIZE_BLOCK) {
-    if (t < ip) raw[t] = tmp[t];
-    out[t] = raw[t];
-  }
-  // repeated convolution with (0.25, 0.5, 0.25), zero beyond the ends (np.convolve 'same'), out and tmp in turn
-  const double* from = out;
-  double* to = tmp;
-  for (int r = 0; r < a.smoothing; ++r) {
-    __syncthreads();
-    for (int t = threadIdx.x; t < T; t += FINALIZE_BLOCK) {
-      double acc;
-      if (t == 0) acc = from[0] * 0.5 + from[1] * 0.25;
-      else if (t == T - 1) acc = from[T - 2] * 0.25 + from[T - 1] * 0.5;
-      else acc = from[t - 1] * 0.25 + from[t] * 0.5 + from[t + 1] * 0.25;
-      to[t] = acc;
-    }
-    double* swap = to;
-    to = const_cast<double*>(from);
-    from = swap;
-  }
-  // the days nearer than `smoothing` to either end keep their own value (also where the two ends overlap)
-  const int sm = std::min(a.smoothing, T);
-  for (int t = threadIdx.x; t < T; t += FINALIZE_BLOCK) {
-    if (t < sm || t >= T - sm) out[t] = raw[t];
-    else if (from != out) out[t] = from[t];
-  }
+  for (int t = threadIdx.x; t < ip; t += FINALIZE_BLOCK) raw[t] = tmp[t];
+  smooth_days(T, a.smoothing, (int)threadIdx.x, FINALIZE_BLOCK, raw, out, tmp, [] { __syncthreads(); });
 }
 
 // numpy 'linear' quantile of a sorted run v[0..n): virtual index (n - 1) q; neighbours floor and

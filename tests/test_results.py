@@ -9,6 +9,9 @@ relative on r_eff (the reference averages float32 dates in float32, the device i
 cvk_reduce equals numpy's quantile / mean / std over the sims.
 """
 
+import os
+import subprocess
+
 import numpy as np
 import pytest
 
@@ -100,6 +103,30 @@ def test_finalize_pop_infected_on_every_variant_row():
     assert np.array_equal(cum[0], 3.0 * np.arange(1, npts + 1) + 7)
     assert np.array_equal(cum[1], np.array([0, 0, 1, 3, 3.0]) + 7)
     assert np.array_equal(cum[2], np.full(npts, 7.0))
+
+
+@pytest.fixture(scope='module')
+def smooth_schedule(tmp_path_factory):
+    """The program that runs the device's smoothing on the CPU, a thread at a time between barriers."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    exe = str(tmp_path_factory.mktemp('smooth') / 'smooth_schedule')
+    subprocess.run(['g++', '-std=c++17', '-O1', '-pthread', '-I', os.path.join(root, 'covasim_amd', 'csrc'), '-o', exe,
+                    os.path.join(root, 'tests', 'golden', 'smooth_schedule.cpp')], check=True)
+    return exe
+
+
+@pytest.mark.parametrize('descending', [0, 1])
+@pytest.mark.parametrize('rounds', [0, 1, 2, 3, 8])
+def test_smoothing_needs_no_luck_in_the_schedule(smooth_schedule, rounds, descending):
+    """However far a thread runs ahead of the others between two barriers, the values are the restatement's."""
+    for npts, threads in [(3, 2), (10, 4), (33, 32), (65, 64)]:
+        raw = np.random.default_rng(npts).uniform(0.5, 2.0, npts)
+        text = f'{npts} {rounds} {threads} {descending}\n' + '\n'.join(f'{x:.17g}' for x in raw)
+        out = subprocess.run([smooth_schedule], input=text, capture_output=True, text=True, check=True, timeout=60).stdout
+        want = rr.smooth(raw, rounds)
+        if rounds:
+            want[:rounds], want[-rounds:] = raw[:rounds], raw[-rounds:]
+        np.testing.assert_allclose([float(x) for x in out.split()], want, rtol=1e-14, atol=0, err_msg=f'{npts} days')
 
 
 # ---------------------------------------------------------------------------------------------
@@ -236,6 +263,38 @@ def test_day_counts_around_waves_and_graph_parts(days):
             assert np.array_equal(res.values, parts.results[key].values, equal_nan=True), key
     want, cvres = oracle_rows(parts)
     assert_rows_match(parts, want, cvres)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('npts', [3, 64, 65, 181, 1100])
+@pytest.mark.parametrize('smoothing', [0, 1, 2, 3, 40])
+def test_r_eff_smoothing_matches_restatement(npts, smoothing):
+    """Every count of smoothing rounds, on days within one wave, across waves and past one workgroup's threads. The
+    16 agents' dates are small whole numbers, so their means are exact; a round is three roundings of positive terms
+    (2^-53 each), 40 rounds and the mean stay below 2^-45."""
+    import torch
+    from covasim_amd import _lib
+    from covasim_amd import results as cvres
+    S, n = 48, 16
+    rng = np.random.default_rng(npts)
+    counts = np.zeros((S, npts, _lib.R_COLS), np.uint32)
+    counts[:, :, _lib.R_COL['new_infections']] = rng.integers(1, 1000, (S, npts))
+    counts[:, :, _lib.R_COL['n_infectious']] = rng.integers(1, 1000, (S, npts))
+    counts_f = np.zeros((S, npts, _lib.RF_COLS))
+    d_inf = rng.integers(0, 20, S * n).astype(np.float32)
+    d_rec = d_inf + 8
+    nan = np.full(S * n, np.nan, np.float32)
+    period = min(npts, 12)
+    dev = lambda a: torch.from_numpy(a).cuda()
+    rows, _ = cvres.finalize_tables(dev(counts.view(np.int32)), dev(counts_f), npts, 1, False, np.zeros(S),
+                                    np.full(S, period), np.arange(S + 1) * n, None, dev(d_inf), dev(d_rec), dev(nan),
+                                    smoothing=smoothing)
+    got = rows[:, cvres.F_ROW_NAMES.index('r_eff')].cpu().numpy()
+    for s in range(S):
+        want = rr.compute_r_eff(counts[s, :, _lib.R_COL['new_infections']].astype(float), np.zeros(npts),
+                                counts[s, :, _lib.R_COL['n_infectious']].astype(float), d_inf[s * n:(s + 1) * n],
+                                d_rec[s * n:(s + 1) * n], nan[:n], period, smoothing)
+        np.testing.assert_allclose(got[s], want, rtol=2.0 ** -45, atol=0, err_msg=f'sim {s}')
 
 
 @pytest.mark.gpu
