@@ -352,7 +352,9 @@ __global__ __launch_bounds__(RELAX_BLOCK) void relax_day_kernel(RelaxDev<R> D, R
       }
       __syncthreads();
     }
-    double c = P != 0.0 ? dP * rcp_d(P) : 0.0;  // at P = 0 the agent cannot escape: its lbar is 0
+    // d log P: below the normal doubles (rcp_d has no reciprocal there) the agent cannot escape, its lbar is at most
+    // 2^-1022 and the sum that c goes into does not hold the product
+    double c = P >= 0x1p-1022 ? dP * rcp_d(P) : 0.0;
 #pragma unroll
     for (int off = 1; off < TPA; off <<= 1) {
       const int other = (int)lane_id() ^ off;

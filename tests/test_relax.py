@@ -407,6 +407,53 @@ def test_relax_ragged_lists_match_cpu_reference(gpu, n, precision):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize('precision', [32, 64])
+@pytest.mark.parametrize('n,lanes', [(0, 4), (200_000, 2)])  # four lanes share an agent's list, or two (n: at least)
+@pytest.mark.parametrize('x,counts', [(5.0, range(49, 57)), (0.9, range(304, 327)), (0.5, range(1018, 1080, 3))])
+def test_relax_escape_below_the_normal_doubles(gpu, precision, n, lanes, x, counts):
+    """Stars whose hub's probability to escape falls, per lane, through the subnormal doubles to zero (1e-6 a saturated
+    contact, 0.1 or 0.5 another): values and gradient are finite and the CPU reference's. Tolerances as for the ragged
+    lists, times the 10 that 1 / (1 - x) amplifies a rounding of x by."""
+    import ctypes as C
+    import torch
+    from covasim_amd import _lib
+    T, f = 3, 0.05
+    sizes = [lanes * k for k in counts]
+    n = max(n, len(sizes) + sum(sizes))
+    pairs, leaf = [], len(sizes)
+    for hub, m in enumerate(sizes):
+        pairs += [(hub, leaf + k) for k in range(m)]
+        leaf += m
+    a = np.array(pairs)
+    tgt, src = np.concatenate([a[:, 0], a[:, 1]]), np.concatenate([a[:, 1], a[:, 0]])
+    order = np.lexsort((src, tgt))
+    indptr = np.concatenate([[0], np.cumsum(np.bincount(tgt, minlength=n))]).astype(np.int64)
+    nbr = src[order].astype(np.int32)
+    bins = (np.arange(n) % 10).astype(np.uint8)
+    rt = np.ones(n, np.float32)
+    w = np.zeros((10, T + 1))
+    w[:, 1] = 1.0  # the seeds' infectiousness on day 1: x
+    w[:, 2] = 0.3
+    theta = np.concatenate([[x / f, 1.0], np.ones(10)])
+    c = np.linspace(1, 2, T)
+    th = torch.tensor(theta, requires_grad=True)
+    e_ref = relax_ref.expected_infections(th, [(indptr, nbr)], bins, rt, w, T, f)
+    (torch.as_tensor(c) * e_ref).sum().backward()
+    dev = [torch.as_tensor(v).cuda() for v in (indptr, nbr, bins, rt)]
+    d = _lib.RelaxDesc(n_agents=n, n_layers=1, n_days=T, kernel_len=T + 1, checkpoint_every=2, precision=precision,
+                       seed_frac=f, age_bin=dev[2].data_ptr(), rel_trans=dev[3].data_ptr(), w_host=w.ctypes.data)
+    d.indptr[0], d.nbr[0] = dev[0].data_ptr(), dev[1].data_ptr()
+    h = C.c_void_p()
+    _lib.check(_lib.lib().cvk_relax_create(C.byref(d), C.byref(h)), 'cvk_relax_create')
+    e, g = _value_and_grad(h, theta, c)
+    assert np.isfinite(e).all() and np.isfinite(g).all()
+    tol = 1000 * (2.0 ** -24 if precision == 32 else 2.0 ** -53)
+    assert _rel(e, e_ref.detach().numpy()) <= tol
+    # x = 5 saturates every contact of every day: the gradient is then exactly zero
+    assert np.linalg.norm(g - th.grad.numpy()) <= tol * np.linalg.norm(th.grad.numpy())
+
+
+@pytest.mark.gpu
 def test_relax_more_agents_than_a_packed_slot_addresses(gpu):
     """2^25 + 3 agents (a slot's layer and bin then travel beside its index), contacts among the last few only: the
     expected infections and gradient are those of the same few agents alone."""
