@@ -113,6 +113,8 @@ def compute_infections(beta, p1, p2, layer_betas, rel_trans, rel_sus, legacy=Fal
     n = rt.numel()
     if rs.numel() != n:
         raise ValueError('rel_trans and rel_sus must have equal lengths')
+    if E and n == 0:  # no array for the device to check the indices against
+        raise IndexError('contact indices outside [0, len(rel_trans))')
     u = None
     if uniforms is not None:
         u, _ = _dev(uniforms, np.float64, 'uniforms')

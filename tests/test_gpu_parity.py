@@ -147,6 +147,21 @@ def test_infections_chunk_edges_match_oracle(gpu, n, E, legacy):
                                         torch.from_numpy(rs).cuda(), legacy=legacy)
 
 
+@pytest.mark.parametrize('host', [False, True])
+def test_infections_of_no_agents(gpu, host):
+    """Contacts among nobody are out of range, as any other index is; no contacts among nobody infect nobody."""
+    import torch
+    import covasim_amd as cv
+    arr = lambda a, dtype: np.asarray(a, dtype) if host else torch.as_tensor(np.asarray(a, dtype)).cuda()
+    nobody = arr([], np.float32)
+    for uniforms in (None, arr(np.full((2, 1), 0.5), np.float64)):
+        with pytest.raises(IndexError):
+            cv.utils.compute_infections(0.3, arr([0], np.int32), arr([0], np.int32), arr([1], np.float32), nobody,
+                                        nobody, uniforms=uniforms)
+    ends = arr([], np.int32)
+    assert [len(x) for x in cv.utils.compute_infections(0.3, ends, ends, nobody, nobody, nobody)] == [0, 0]
+
+
 def run_pair(pop, n_days=40, seed=1, variants=(), use_graph=None, **pars):
     import covasim_amd as cv
     gpars = dict(pars)
