@@ -149,7 +149,8 @@ __global__ __launch_bounds__(INF_BLOCK) void infections_scan_kernel(InfArgs a) {
   uint16_t* queue = (uint16_t*)area;  // edge of the chunk | dir 0 << 9 | dir 1 << 10
   uint32_t* s_hit = area + INF_CHUNK / 2;
   const uint32_t lane = inf_lane();
-  const uint32_t n = (uint32_t)a.n_agents, nm1 = n ? n - 1u : 0u;
+  // no index is above 2^31 - 1 (and a negative one is, taken as unsigned)
+  const uint32_t n = a.n_agents < ((int64_t)1 << 31) ? (uint32_t)a.n_agents : 1u << 31, nm1 = n ? n - 1u : 0u;
   int64_t c0, c1;
   inf_range(a, c0, c1);
   uint32_t mine = 0, bad = 0;

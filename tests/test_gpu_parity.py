@@ -162,6 +162,27 @@ def test_infections_of_no_agents(gpu, host):
     assert [len(x) for x in cv.utils.compute_infections(0.3, ends, ends, nobody, nobody, nobody)] == [0, 0]
 
 
+def test_infections_of_more_agents_than_32_bits_count(gpu):
+    """2^32 + 5 agents: an index is checked against all of them (a negative one is still refused), and the infections
+    are those among the agents that the contacts name."""
+    import torch
+    import covasim_amd as cv
+    named, E, n = 1000, 3000, 2 ** 32 + 5
+    rng = np.random.default_rng(8)
+    ends = [torch.as_tensor(rng.integers(0, named, E).astype(np.int32)).cuda() for _ in range(2)]
+    betas = torch.ones(E, device='cuda')
+    factor = torch.zeros(n, device='cuda')
+    factor[:named] = torch.as_tensor(rng.random(named).astype(np.float32)).cuda()
+    cv.utils.set_seed(12)
+    got = cv.utils.compute_infections(0.9, *ends, betas, factor, factor, return_probs=True)
+    few = factor[:named].clone()
+    want = cv.utils.compute_infections(0.9, *ends, betas, few, few, return_probs=True)
+    assert len(want[0]) > 100 and all(torch.equal(g, w) for g, w in zip(got, want))
+    ends[0][7] = -1
+    with pytest.raises(IndexError):
+        cv.utils.compute_infections(0.9, *ends, betas, factor, factor)
+
+
 def run_pair(pop, n_days=40, seed=1, variants=(), use_graph=None, **pars):
     import covasim_amd as cv
     gpars = dict(pars)
