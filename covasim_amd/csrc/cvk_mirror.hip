@@ -267,6 +267,7 @@ __global__ __launch_bounds__(INF_BLOCK) void infections_write_kernel(InfArgs a, 
     for (int k = 0; k < INF_WAVES; ++k) v[q] += s_sum[k][q];
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) a.out[0] = v[0] + v[1];
+  if ((int64_t)(v[0] + v[1]) > capacity || a.out[1]) return;  // refused: the outputs stay as they were (uniform)
   int64_t c0, c1;
   inf_range(a, c0, c1);
   const unsigned long long start0 = v[2], start1 = v[0] + v[3];

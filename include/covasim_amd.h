@@ -325,8 +325,8 @@ int cvk_trans_sus(const float* rel_trans, const float* rel_sus, const uint8_t* i
  * uniforms: NULL for counter-based Philox draws keyed by (seed, t, variant, layer), else a
  * device float64 array [2][n_edges] of per-(direction, edge) uniforms. prob_out (may be NULL)
  * receives the float32 probability of each emitted pair. *count_host receives the number of
- * pairs; returns CVK_E_CAPACITY (after writing count) if it exceeds capacity. Synchronises
- * the stream to read the count. */
+ * pairs; returns CVK_E_CAPACITY (after writing count) if it exceeds capacity. A refused call writes no
+ * pair. Synchronises the stream to read the count. */
 int cvk_infections(float beta, const int32_t* p1, const int32_t* p2, const float* layer_betas,
                    int64_t n_edges, const float* rel_trans, const float* rel_sus, int64_t n_agents,
                    const double* uniforms, uint64_t seed, int32_t t, int32_t variant, int32_t layer,

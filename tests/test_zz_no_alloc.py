@@ -81,3 +81,30 @@ def test_noalloc_errors(gpu):
     c = call('cvk_infections_noalloc', 0.9, p1, p2, lb, rt, rs)
     d = call('cvk_infections', 0.9, p1, p2, lb, rt, rs)
     assert c[1] == d[1] and all(np.array_equal(x, y) for x, y in zip(c[2:], d[2:]))
+
+
+@pytest.mark.parametrize('entry', ['cvk_infections', 'cvk_infections_noalloc', 'cvk_infections_work'])
+def test_refused_calls_leave_the_outputs_alone(gpu, entry):
+    """One pair too many for the outputs, or an index outside the population: an error, and nothing written."""
+    import torch
+    from covasim_amd import _lib
+    L = _lib.lib()
+    p1, p2, lb, rt, rs, _ = inputs(4, 3000, 40_000)
+    E, n = p1.numel(), rt.numel()
+    work = torch.empty(L.cvk_infections_work_bytes(E, n), dtype=torch.uint8, device='cuda')
+    outs = [torch.full((2 * E,), -7, dtype=torch.int32, device='cuda') for _ in range(2)]
+    prob = torch.full((2 * E,), -1.0, device='cuda')
+
+    def refused(capacity):
+        count = C.c_int64(-1)
+        extra = (None, work.data_ptr(), work.numel()) if entry.endswith('work') else ()
+        rc = getattr(L, entry)(0.9, p1.data_ptr(), p2.data_ptr(), lb.data_ptr(), E, rt.data_ptr(), rs.data_ptr(), n,
+                               None, 77, 0, 0, 0, 0, outs[0].data_ptr(), outs[1].data_ptr(), prob.data_ptr(), capacity,
+                               C.byref(count), *extra, _lib.stream_ptr())
+        torch.cuda.synchronize()
+        return rc, count.value, int((outs[0] != -7).sum() + (outs[1] != -7).sum() + (prob != -1).sum())
+    total = call('cvk_infections', 0.9, p1, p2, lb, rt, rs)[1]
+    assert total > 1000
+    assert refused(total - 1) == (_lib.E_CAPACITY, total, 0)
+    p2[E // 2] = n
+    assert refused(2 * E) == (_lib.E_INVALID, 0, 0)
