@@ -71,6 +71,9 @@ __global__ void trans_sus_kernel(const float* __restrict__ rel_trans, const floa
 // gathered rel_trans at both ends of every edge and drew a Philox block per slot with a nonzero source, with one
 // workgroup scanning the counts between them: 129 + 149 + 21 us at 1M agents and 10M edges, 5 % of them
 // infectious, against 4 + 50 + 15 us. (The next chunk's columns loaded ahead of the candidates: 55 us.)
+// cvk_infections_noalloc, whose scratch is fixed, keeps the waves' counts and a flag for each chunk: its writing pass
+// finds the hits of the flagged chunks anew (213 us at the sizes above with 4050 pairs; 181 with a hit bit for
+// every slot, which took 16 MiB of every process on every GPU; 302 without the flags).
 // ---------------------------------------------------------------------------
 struct InfArgs {
   float beta;
@@ -89,7 +92,9 @@ struct InfArgs {
   uint64_t* bits;      // one bit per agent, 16-byte aligned and padded (null: rel_trans itself is gathered)
   int32_t lds_words;   // 32-bit words of it staged in LDS, or 0: read from memory
   int64_t chunks;
-  uint32_t* hits;      // [2][chunks][16] hit bits
+  uint32_t* hits;      // [2][chunks][16] hit bits (null: not kept, the writing pass finds them anew)
+  uint8_t* flags;      // with hits null: [n_flags] whether chunk c has any; chunks from n_flags on are always searched
+  int64_t n_flags;
   uint32_t* cnt;       // [2][waves] hits of each wave
   uint64_t* out;       // [2] the total, and nonzero if an endpoint is outside [0, n_agents)
 };
@@ -136,98 +141,118 @@ __device__ inline void inf_range(const InfArgs& a, int64_t& c0, int64_t& c1) {
   c1 = a.chunks * (w + 1) / W;
 }
 
+// Hit bits of chunk c into s_hit (16 words a direction; wave-wide, the words and the queue are this wave's): whether
+// this lane met an endpoint outside the population.
+template <int MODE>
+__device__ inline uint32_t inf_chunk_hits(const InfArgs& a, int64_t c, const uint32_t* map, uint16_t* queue, uint32_t* s_hit) {
+  const uint32_t lane = inf_lane();
+  // no index is above 2^31 - 1 (and a negative one is, taken as unsigned)
+  const uint32_t n = a.n_agents < ((int64_t)1 << 31) ? (uint32_t)a.n_agents : 1u << 31, nm1 = n ? n - 1u : 0u;
+  uint32_t bad = 0;
+  const int64_t e0 = c * INF_CHUNK;
+  uint32_t x[INF_K], y[INF_K];
+#pragma unroll
+  for (int k = 0; k < INF_K; ++k) {
+    const int64_t e = e0 + k * 64 + lane;
+    x[k] = e < a.n_edges ? (uint32_t)a.p1[e] : 0u;
+    y[k] = e < a.n_edges ? (uint32_t)a.p2[e] : 0u;
+  }
+  uint32_t f1 = 0, f2 = 0;  // bit k: the direction's source can transmit
+#pragma unroll
+  for (int k = 0; k < INF_K; ++k) {
+    const bool in = e0 + k * 64 + lane < a.n_edges;
+    const bool ok = in && x[k] < n && y[k] < n;
+    bad |= in && !ok ? 1u : 0u;
+    const uint32_t xs = x[k] < nm1 ? x[k] : nm1, ys = y[k] < nm1 ? y[k] : nm1;
+    bool s1 = false, s2 = false;
+    if (ok) {
+      if (MODE == INF_DIRECT) {
+        s1 = !(a.rel_trans[xs] == 0.0f);
+        s2 = !(a.rel_trans[ys] == 0.0f);
+      } else {
+        const uint32_t* words = MODE == INF_LDS ? map : (const uint32_t*)a.bits;
+        s1 = (words[xs >> 5] >> (xs & 31u)) & 1u;
+        s2 = (words[ys >> 5] >> (ys & 31u)) & 1u;
+      }
+    }
+    f1 |= (uint32_t)s1 << k;
+    f2 |= (uint32_t)(s2 && a.dirs == 2) << k;
+  }
+  uint32_t n_q = 0;
+  inf_wave_sync();  // the previous chunk's words have been read
+#pragma unroll
+  for (int k = 0; k < INF_K; ++k) {
+    const bool cand = ((f1 | f2) >> k) & 1u;
+    const uint64_t m = __ballot(cand);
+    if (cand) queue[n_q + inf_below(m)] = (uint16_t)((k * 64 + lane) | (((f1 >> k) & 1u) << 9) | (((f2 >> k) & 1u) << 10));
+    n_q += (uint32_t)__popcll(m);
+  }
+  if (lane < 2 * INF_CHUNK_WORDS) s_hit[lane] = 0;
+  inf_wave_sync();
+  for (uint32_t r = 0; r < n_q; r += 64) {  // wave-uniform
+    if (r + lane < n_q) {
+      const uint32_t q = queue[r + lane], j = q & (INF_CHUNK - 1);
+      const int64_t e = e0 + j;
+      const int32_t xe = a.p1[e], ye = a.p2[e];
+      const float bl = a.beta * a.layer_betas[e];
+      float p[2] = {0.0f, 0.0f};
+      if (q & (1u << 9)) p[0] = (bl * a.rel_trans[xe]) * a.rel_sus[ye];   // :117
+      if (q & (1u << 10)) p[1] = (bl * a.rel_trans[ye]) * a.rel_sus[xe];
+      if (p[0] != 0.0f || p[1] != 0.0f) {                                 // :118
+        double u[2];
+        if (a.uniforms) {
+          u[0] = a.uniforms[e];
+          u[1] = p[1] != 0.0f ? a.uniforms[a.n_edges + e] : 1.0;
+        } else {
+          const uint64_t ue = (uint64_t)e;
+          const u32x4 w = philox_seeded(a.seed, (uint32_t)ue, (uint32_t)a.t,
+                                        STREAM_TX | ((uint32_t)a.variant << 8) | (uint32_t)a.layer, (uint32_t)(ue >> 32));
+          u[0] = u01(w.x, w.y);
+          u[1] = u01(w.z, w.w);
+        }
+#pragma unroll
+        for (int d = 0; d < 2; ++d)
+          if (p[d] != 0.0f && u[d] < (double)p[d])                        // :123
+            atomicOr(&s_hit[d * INF_CHUNK_WORDS + (j >> 5)], 1u << (j & 31u));
+      }
+    }
+  }
+  inf_wave_sync();
+  return bad;
+}
+
+// This wave's part of the dynamic LDS after lds_words words of bitmap: the queue (edge of the chunk | dir 0 << 9 |
+// dir 1 << 10) and the hit words.
+__device__ inline void inf_wave_area(uint32_t* s_inf, int32_t lds_words, uint16_t** queue, uint32_t** s_hit) {
+  uint32_t* area = s_inf + lds_words + (threadIdx.x >> 6) * INF_WAVE_WORDS;
+  *queue = (uint16_t*)area;
+  *s_hit = area + INF_CHUNK / 2;
+}
+
 template <int MODE>
 __global__ __launch_bounds__(INF_BLOCK) void infections_scan_kernel(InfArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint32_t s_inf[];
-  const uint32_t* map = s_inf;
   if (MODE == INF_LDS) {
     const uint4* src = (const uint4*)a.bits;
     for (int j = threadIdx.x; j < (a.lds_words >> 2); j += INF_BLOCK) ((uint4*)s_inf)[j] = src[j];
     __syncthreads();
   }
-  uint32_t* area = s_inf + (MODE == INF_LDS ? a.lds_words : 0) + (threadIdx.x >> 6) * INF_WAVE_WORDS;
-  uint16_t* queue = (uint16_t*)area;  // edge of the chunk | dir 0 << 9 | dir 1 << 10
-  uint32_t* s_hit = area + INF_CHUNK / 2;
+  uint16_t* queue;
+  uint32_t* s_hit;
+  inf_wave_area(s_inf, MODE == INF_LDS ? a.lds_words : 0, &queue, &s_hit);
   const uint32_t lane = inf_lane();
-  // no index is above 2^31 - 1 (and a negative one is, taken as unsigned)
-  const uint32_t n = a.n_agents < ((int64_t)1 << 31) ? (uint32_t)a.n_agents : 1u << 31, nm1 = n ? n - 1u : 0u;
   int64_t c0, c1;
   inf_range(a, c0, c1);
   uint32_t mine = 0, bad = 0;
   for (int64_t c = c0; c < c1; ++c) {  // wave-uniform
-    const int64_t e0 = c * INF_CHUNK;
-    uint32_t x[INF_K], y[INF_K];
-#pragma unroll
-    for (int k = 0; k < INF_K; ++k) {
-      const int64_t e = e0 + k * 64 + lane;
-      x[k] = e < a.n_edges ? (uint32_t)a.p1[e] : 0u;
-      y[k] = e < a.n_edges ? (uint32_t)a.p2[e] : 0u;
-    }
-    uint32_t f1 = 0, f2 = 0;  // bit k: the direction's source can transmit
-#pragma unroll
-    for (int k = 0; k < INF_K; ++k) {
-      const bool in = e0 + k * 64 + lane < a.n_edges;
-      const bool ok = in && x[k] < n && y[k] < n;
-      bad |= in && !ok ? 1u : 0u;
-      const uint32_t xs = x[k] < nm1 ? x[k] : nm1, ys = y[k] < nm1 ? y[k] : nm1;
-      bool s1 = false, s2 = false;
-      if (ok) {
-        if (MODE == INF_DIRECT) {
-          s1 = !(a.rel_trans[xs] == 0.0f);
-          s2 = !(a.rel_trans[ys] == 0.0f);
-        } else {
-          const uint32_t* words = MODE == INF_LDS ? map : (const uint32_t*)a.bits;
-          s1 = (words[xs >> 5] >> (xs & 31u)) & 1u;
-          s2 = (words[ys >> 5] >> (ys & 31u)) & 1u;
-        }
-      }
-      f1 |= (uint32_t)s1 << k;
-      f2 |= (uint32_t)(s2 && a.dirs == 2) << k;
-    }
-    uint32_t n_q = 0;
-    inf_wave_sync();  // the previous chunk's words have been read
-#pragma unroll
-    for (int k = 0; k < INF_K; ++k) {
-      const bool cand = ((f1 | f2) >> k) & 1u;
-      const uint64_t m = __ballot(cand);
-      if (cand) queue[n_q + inf_below(m)] = (uint16_t)((k * 64 + lane) | (((f1 >> k) & 1u) << 9) | (((f2 >> k) & 1u) << 10));
-      n_q += (uint32_t)__popcll(m);
-    }
-    if (lane < 2 * INF_CHUNK_WORDS) s_hit[lane] = 0;
-    inf_wave_sync();
-    for (uint32_t r = 0; r < n_q; r += 64) {  // wave-uniform
-      if (r + lane < n_q) {
-        const uint32_t q = queue[r + lane], j = q & (INF_CHUNK - 1);
-        const int64_t e = e0 + j;
-        const int32_t xe = a.p1[e], ye = a.p2[e];
-        const float bl = a.beta * a.layer_betas[e];
-        float p[2] = {0.0f, 0.0f};
-        if (q & (1u << 9)) p[0] = (bl * a.rel_trans[xe]) * a.rel_sus[ye];   // :117
-        if (q & (1u << 10)) p[1] = (bl * a.rel_trans[ye]) * a.rel_sus[xe];
-        if (p[0] != 0.0f || p[1] != 0.0f) {                                 // :118
-          double u[2];
-          if (a.uniforms) {
-            u[0] = a.uniforms[e];
-            u[1] = p[1] != 0.0f ? a.uniforms[a.n_edges + e] : 1.0;
-          } else {
-            const uint64_t ue = (uint64_t)e;
-            const u32x4 w = philox_seeded(a.seed, (uint32_t)ue, (uint32_t)a.t,
-                                          STREAM_TX | ((uint32_t)a.variant << 8) | (uint32_t)a.layer, (uint32_t)(ue >> 32));
-            u[0] = u01(w.x, w.y);
-            u[1] = u01(w.z, w.w);
-          }
-#pragma unroll
-          for (int d = 0; d < 2; ++d)
-            if (p[d] != 0.0f && u[d] < (double)p[d])                        // :123
-              atomicOr(&s_hit[d * INF_CHUNK_WORDS + (j >> 5)], 1u << (j & 31u));
-        }
-      }
-    }
-    inf_wave_sync();
-    if (lane < (uint32_t)(a.dirs * INF_CHUNK_WORDS)) {
-      const uint32_t h = s_hit[lane];
+    bad |= inf_chunk_hits<MODE>(a, c, s_inf, queue, s_hit);
+    const uint32_t h = lane < (uint32_t)(a.dirs * INF_CHUNK_WORDS) ? s_hit[lane] : 0u;
+    mine += (uint32_t)__popc(h);
+    if (!a.hits) {  // uniform
+      const bool any = __ballot(h != 0) != 0;
+      if (lane == 0 && c < a.n_flags) a.flags[c] = any ? 1 : 0;
+    } else if (lane < (uint32_t)(a.dirs * INF_CHUNK_WORDS)) {
       a.hits[((int64_t)(lane / INF_CHUNK_WORDS) * a.chunks + c) * INF_CHUNK_WORDS + lane % INF_CHUNK_WORDS] = h;
-      mine += (uint32_t)__popc(h);
     }
   }
   const uint32_t n0 = inf_wave_sum(lane < INF_CHUNK_WORDS ? mine : 0u), n1 = inf_wave_sum(lane < INF_CHUNK_WORDS ? 0u : mine);
@@ -239,9 +264,15 @@ __global__ __launch_bounds__(INF_BLOCK) void infections_scan_kernel(InfArgs a) {
   if (__ballot(bad != 0) && lane == 0) a.out[1] = 1;
 }
 
-// Same grid as the scan.
-__global__ __launch_bounds__(INF_BLOCK) void infections_write_kernel(InfArgs a, int64_t capacity, int32_t* src_out,
-                                                                     int32_t* tgt_out, float* prob_out) {
+struct InfOut {
+  int64_t capacity;
+  int32_t *src, *tgt;
+  float* prob;  // may be null
+};
+
+// Position of this wave's first pair of each direction, from the scan's counts (same grid); block 0 keeps the total.
+// False, for the whole grid, where the call is refused: the outputs then stay as they were. Block-wide.
+__device__ inline bool inf_positions(const InfArgs& a, const InfOut& o, uint64_t (&pos)[2]) {
   __shared__ unsigned long long s_sum[INF_WAVES][4];
   const uint32_t lane = inf_lane(), wave = threadIdx.x >> 6;
   const int W = (int)gridDim.x * INF_WAVES, first = (int)blockIdx.x * INF_WAVES;
@@ -267,38 +298,82 @@ __global__ __launch_bounds__(INF_BLOCK) void infections_write_kernel(InfArgs a, 
     for (int k = 0; k < INF_WAVES; ++k) v[q] += s_sum[k][q];
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) a.out[0] = v[0] + v[1];
-  if ((int64_t)(v[0] + v[1]) > capacity || a.out[1]) return;  // refused: the outputs stay as they were (uniform)
+  if ((int64_t)(v[0] + v[1]) > o.capacity || a.out[1]) return false;
+  pos[0] = v[2];
+  pos[1] = v[0] + v[3];
+  for (int d = 0; d < a.dirs; ++d)
+    for (uint32_t k = 0; k < wave; ++k) pos[d] += a.cnt[d * W + first + (int)k];
+  return true;
+}
+
+// Writes the pairs of hit word h (edges e0 .. e0 + 31 in direction d) from position at on.
+__device__ inline void inf_write_word(const InfArgs& a, const InfOut& o, uint32_t h, int64_t e0, int d, int64_t at) {
+  while (h) {
+    const int64_t e = e0 + (__ffs(h) - 1);
+    h &= h - 1;
+    const int32_t x = a.p1[e], y = a.p2[e];
+    const int32_t src = d ? y : x, tgt = d ? x : y;
+    if (at < o.capacity) {
+      o.src[at] = src;
+      o.tgt[at] = tgt;
+      if (o.prob) o.prob[at] = ((a.beta * a.layer_betas[e]) * a.rel_trans[src]) * a.rel_sus[tgt];
+    }
+    ++at;
+  }
+}
+
+// Same grid as the scan.
+__global__ __launch_bounds__(INF_BLOCK) void infections_write_kernel(InfArgs a, InfOut o) {
+  const uint32_t lane = inf_lane();
+  uint64_t start[2];
+  if (!inf_positions(a, o, start)) return;
   int64_t c0, c1;
   inf_range(a, c0, c1);
-  const unsigned long long start0 = v[2], start1 = v[0] + v[3];
   for (int d = 0; d < a.dirs; ++d) {
-    uint64_t pos = d ? start1 : start0;
-    for (uint32_t k = 0; k < wave; ++k) pos += a.cnt[d * W + first + (int)k];
+    uint64_t pos = start[d];
     const uint32_t* hits = a.hits + (int64_t)d * a.chunks * INF_CHUNK_WORDS;
     for (int64_t w0 = c0 * INF_CHUNK_WORDS; w0 < c1 * INF_CHUNK_WORDS; w0 += 64) {  // wave-uniform
-      uint32_t h = w0 + lane < c1 * INF_CHUNK_WORDS ? hits[w0 + lane] : 0u;
+      const uint32_t h = w0 + lane < c1 * INF_CHUNK_WORDS ? hits[w0 + lane] : 0u;
       const uint32_t cnt = (uint32_t)__popc(h);
       uint32_t incl = cnt;
 #pragma unroll
       for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t o = __shfl_up(incl, off, 64);
-        if ((int)lane >= off) incl += o;
+        const uint32_t o2 = __shfl_up(incl, off, 64);
+        if ((int)lane >= off) incl += o2;
       }
-      int64_t at = (int64_t)(pos + incl - cnt);
-      while (h) {
-        const int64_t e = (w0 + lane) * 32 + (__ffs(h) - 1);
-        h &= h - 1;
-        const int32_t x = a.p1[e], y = a.p2[e];
-        const int32_t src = d ? y : x, tgt = d ? x : y;
-        if (at < capacity) {
-          src_out[at] = src;
-          tgt_out[at] = tgt;
-          if (prob_out) prob_out[at] = ((a.beta * a.layer_betas[e]) * a.rel_trans[src]) * a.rel_sus[tgt];
-        }
-        ++at;
-      }
+      inf_write_word(a, o, h, (w0 + lane) * 32, d, (int64_t)(pos + incl - cnt));
       pos += __shfl(incl, 63, 64);
     }
+  }
+}
+
+// The same where the scan's hit bits were not kept (same grid): a flagged chunk's are found again, then written out.
+__global__ __launch_bounds__(INF_BLOCK) void infections_rescan_kernel(InfArgs a, InfOut o) {
+  extern __shared__ __attribute__((aligned(16))) uint32_t s_inf[];
+  uint16_t* queue;
+  uint32_t* s_hit;
+  inf_wave_area(s_inf, 0, &queue, &s_hit);
+  const uint32_t lane = inf_lane();
+  uint64_t pos[2];
+  if (!inf_positions(a, o, pos)) return;
+  int64_t c0, c1;
+  inf_range(a, c0, c1);
+  const int d = lane / INF_CHUNK_WORDS;  // lanes 0 .. 15 hold direction 0's words, 16 .. 31 direction 1's
+  static_assert(INF_CHUNK_WORDS == 16, "a direction's words are a group of 16 lanes");
+  for (int64_t c = c0; c < c1; ++c) {  // wave-uniform
+    if (c < a.n_flags && !a.flags[c]) continue;
+    (void)inf_chunk_hits<INF_DIRECT>(a, c, s_inf, queue, s_hit);
+    const uint32_t h = d < a.dirs ? s_hit[lane] : 0u;
+    const uint32_t cnt = (uint32_t)__popc(h);
+    uint32_t incl = cnt;
+#pragma unroll
+    for (int off = 1; off < INF_CHUNK_WORDS; off <<= 1) {
+      const uint32_t o2 = __shfl_up(incl, off, INF_CHUNK_WORDS);
+      if ((int)(lane % INF_CHUNK_WORDS) >= off) incl += o2;
+    }
+    inf_write_word(a, o, h, c * INF_CHUNK + (int64_t)(lane % INF_CHUNK_WORDS) * 32, d, (int64_t)((d ? pos[1] : pos[0]) + incl - cnt));
+    pos[0] += __shfl(incl, INF_CHUNK_WORDS - 1, 64);
+    pos[1] += __shfl(incl, 2 * INF_CHUNK_WORDS - 1, 64);
   }
 }
 
@@ -394,8 +469,9 @@ static int infections_args(InfArgs& a, float beta, const int32_t* p1, const int3
   return CVK_OK;
 }
 
-// Runs the three launches; a's scratch pointers are set (a.bits may be null: rel_trans itself is gathered). Reads the
-// total back; *outside (if given) receives whether an endpoint lies outside [0, n_agents), an error otherwise.
+// Runs the three launches; a's scratch pointers are set (a.bits and a.hits may both be null: rel_trans itself is
+// gathered, and the hits are found twice). Reads the total back; *outside (if given) receives whether an endpoint lies
+// outside [0, n_agents), an error otherwise.
 static int infections_run(InfArgs a, int32_t* src_out, int32_t* tgt_out, float* prob_out, int64_t capacity,
                           int64_t* count_host, int32_t* outside, hipStream_t st, const char* name) {
   int64_t budget = 0;
@@ -411,7 +487,9 @@ static int infections_run(InfArgs a, int32_t* src_out, int32_t* tgt_out, float* 
   const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>(std::min(n_cu, INF_MAX_GRID), a.chunks));
   const auto scan = !a.bits ? infections_scan_kernel<INF_DIRECT> : in_lds ? infections_scan_kernel<INF_LDS> : infections_scan_kernel<INF_L2>;
   hipLaunchKernelGGL(scan, dim3(grid), dim3(INF_BLOCK), (size_t)((in_lds ? bits : 0) + queues), st, a);
-  hipLaunchKernelGGL(infections_write_kernel, dim3(grid), dim3(INF_BLOCK), 0, st, a, capacity, src_out, tgt_out, prob_out);
+  const InfOut o = {capacity, src_out, tgt_out, prob_out};
+  if (a.hits) hipLaunchKernelGGL(infections_write_kernel, dim3(grid), dim3(INF_BLOCK), 0, st, a, o);
+  else hipLaunchKernelGGL(infections_rescan_kernel, dim3(grid), dim3(INF_BLOCK), (size_t)queues, st, a, o);
   rc = check_launch(name);
   if (rc) return rc;
   uint64_t out[2] = {0, 0};
@@ -476,12 +554,14 @@ extern "C" int cvk_infections(float beta, const int32_t* p1, const int32_t* p2, 
 }
 
 // ---- the same computation without allocation ----
-// Scratch of cvk_infections_noalloc: the total, the waves' counts and the hit bits of the most slots it takes (16 MiB;
-// there is no room for a bit per agent of any population, so its scan gathers rel_trans itself). Every GPU the
-// library runs on holds its own copy until the process ends. In host code `scratch` only names the symbol; its device
-// address comes from hipGetSymbolAddress, once per device, and only that address is passed to kernels.
-constexpr int64_t NOALLOC_HIT_WORDS = CVK_INFECTIONS_NOALLOC_MAX_SLOTS / 32 + 2 * INF_CHUNK_WORDS;
-static __device__ __align__(256) uint32_t scratch[4 + INF_CNT_WORDS + NOALLOC_HIT_WORDS];
+// Scratch of cvk_infections_noalloc: the total, the waves' counts and, in the rest of 256 KiB, the chunks' flags (all
+// but the last 32784 chunks of the largest legacy call). There is no room for a bit per agent of any population or per
+// slot, so its scan gathers rel_trans itself and its writing pass finds the hits anew: nothing that one call leaves
+// here is an index to another. Every GPU the library runs on holds its own copy until the process ends. In host code
+// `scratch` only names the symbol; its device address comes from hipGetSymbolAddress, once per device, and only that
+// address is passed to kernels.
+constexpr int64_t SCRATCH_WORDS = 65536;  // the size the header gives
+static __device__ __align__(256) uint32_t scratch[SCRATCH_WORDS];
 
 namespace {
 constexpr int kMaxDevices = 64;
@@ -526,7 +606,8 @@ extern "C" int cvk_infections_noalloc(float beta, const int32_t* p1, const int32
   if (rc != CVK_OK) return rc;
   a.out = (uint64_t*)base;
   a.cnt = base + 4;
-  a.hits = base + 4 + INF_CNT_WORDS;
+  a.flags = (uint8_t*)(base + 4 + INF_CNT_WORDS);
+  a.n_flags = (SCRATCH_WORDS - 4 - INF_CNT_WORDS) * 4;
   return infections_run(a, src_out, tgt_out, prob_out, capacity, count_host, nullptr, (hipStream_t)stream,
                         "cvk_infections_noalloc");
 }

@@ -345,7 +345,7 @@ int cvk_infections_work(float beta, const int32_t* p1, const int32_t* p2, const 
 
 /* No reference counterpart: cvk_infections without any allocation, for callers that cannot call
  * hipMalloc (serving loops, harnesses that forbid allocation). Same arguments, results and errors
- * as cvk_infections; its scratch is a fixed device array of the library (16 MiB per
+ * as cvk_infections; its scratch is a fixed device array of the library (256 KiB per
  * GPU, held until the process ends) instead of a per-call allocation. Limit: at most
  * CVK_INFECTIONS_NOALLOC_MAX_SLOTS edge slots (2 * n_edges, or n_edges with legacy != 0); larger
  * calls return CVK_E_CAPACITY before any device work. Calls that overlap on one GPU (two host

@@ -165,3 +165,21 @@ def test_noalloc_limit_matches_header():
     chunk = int(re.search(r'#define CVK_INFECTIONS_NOALLOC_MAX_SLOTS \(CVK_INFECTIONS_NOALLOC_MAX_BLOCKS \* (\d+)LL\)',
                           hdr).group(1))
     assert _lib.INFECTIONS_NOALLOC_MAX_SLOTS == blocks * chunk
+
+
+def test_library_holds_little_static_memory():
+    """The library's arrays, on every GPU and as their shadow here: hardly more than the 256 KiB that the header gives
+    for cvk_infections_noalloc's."""
+    import struct
+
+    from covasim_amd import _lib
+    data = open(_lib.lib()._name, 'rb').read()
+    assert data[:5] == b'\x7fELF\x02'
+    offset, = struct.unpack_from('<Q', data, 40)
+    entry, count = struct.unpack_from('<HH', data, 58)
+    nobits = 0
+    for k in range(count):
+        kind, = struct.unpack_from('<I', data, offset + k * entry + 4)
+        size, = struct.unpack_from('<Q', data, offset + k * entry + 32)
+        nobits += size if kind == 8 else 0
+    assert 256 << 10 <= nobits <= 272 << 10

@@ -83,6 +83,36 @@ def test_noalloc_errors(gpu):
     assert c[1] == d[1] and all(np.array_equal(x, y) for x, y in zip(c[2:], d[2:]))
 
 
+@pytest.mark.parametrize('legacy', [0, 1])
+@pytest.mark.parametrize('E', [1, 31, 32, 511, 512, 513, 4096 * 512 - 1, 4096 * 512 + 1])
+def test_noalloc_chunk_edges(gpu, E, legacy):
+    """Edge counts at and around a word of hits, a chunk, and a chunk for every wave of the launch: the pairs of the
+    writing pass that finds the hits anew are, in their order, those of the one that kept them."""
+    p1, p2, lb, rt, rs, U = inputs(E, max(20, E // 50), max(E, 20))
+    p1, p2, lb, U = p1[:E].clone(), p2[:E].clone(), lb[:E].clone(), U[:, :E].contiguous()
+    for uni in (None, U):
+        a = call('cvk_infections', 0.9, p1, p2, lb, rt, rs, uni, legacy, t=3, v=1, l=2)
+        b = call('cvk_infections_noalloc', 0.9, p1, p2, lb, rt, rs, uni, legacy, t=3, v=1, l=2)
+        assert a[:2] == b[:2] and all(np.array_equal(x, y) for x, y in zip(a[2:], b[2:]))
+        assert a[1] > 0 or E < 512
+
+
+@pytest.mark.parametrize('legacy', [0, 1])
+def test_noalloc_largest_call(gpu, legacy):
+    """As many slots as it takes; with legacy the last chunks are past those that the scratch has a flag for."""
+    import torch
+    from covasim_amd import _lib
+    n, E = 100_000, _lib.INFECTIONS_NOALLOC_MAX_SLOTS // (1 if legacy else 2)
+    g = torch.Generator(device='cuda').manual_seed(5)
+    p1, p2 = torch.randint(0, n, (2, E), generator=g, device='cuda', dtype=torch.int32)
+    rt = torch.zeros(n, device='cuda')
+    rt[:100] = 0.5
+    lb, rs = torch.ones(E, device='cuda'), torch.ones(n, device='cuda')
+    a = call('cvk_infections', 0.5, p1, p2, lb, rt, rs, legacy=legacy)
+    b = call('cvk_infections_noalloc', 0.5, p1, p2, lb, rt, rs, legacy=legacy)
+    assert a[:2] == b[:2] and a[1] > 1000 and all(np.array_equal(x, y) for x, y in zip(a[2:], b[2:]))
+
+
 @pytest.mark.parametrize('entry', ['cvk_infections', 'cvk_infections_noalloc', 'cvk_infections_work'])
 def test_refused_calls_leave_the_outputs_alone(gpu, entry):
     """One pair too many for the outputs, or an index outside the population: an error, and nothing written."""
