@@ -373,8 +373,8 @@ def run_relax(w, args):
     truth_sim = make_sim(args.seed)
     truth_sim.run()
     observed = truth_sim.results['new_infections'].values.copy()
-    r32 = Relaxation(make_sim(args.seed), precision=32, checkpoint_every=10)
-    r64 = Relaxation(r32.sim, precision=64, checkpoint_every=10)
+    r32 = Relaxation(make_sim(args.seed), precision=32)
+    r64 = Relaxation(r32.sim, precision=64)
     setup_s = time.perf_counter() - t0
     theta = r32.theta0()
     c = np.random.default_rng(args.seed).uniform(0.5, 1.5, r32.n_days) / 1e4

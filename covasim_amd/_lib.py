@@ -232,6 +232,9 @@ class BatchConfig(C.Structure):
         return (self.edge_block, self.edge_chunks, self.edge_blocks_per_cu, self.agents_per_thread)
 
 
+RELAX_ALL_DAYS = -1  # segment_days: every day's record held, where they fit
+
+
 class RelaxDesc(C.Structure):
     _fields_ = [('n_agents', C.c_int64), ('n_layers', C.c_int32), ('n_days', C.c_int32), ('kernel_len', C.c_int32),
                 ('checkpoint_every', C.c_int32), ('precision', C.c_int32), ('segment_days', C.c_int32),

@@ -11,8 +11,11 @@ a differentiable torch function of theta = [beta, beta_layer for each layer, rel
 the 10 prognosis age bins]. The model and its adjoint are spelled out in
 ``csrc/cvk_relax.hip``. The forward runs in float32 (precision=32, log-space products
 accumulated in float32) or float64 (precision=64). The gradient comes from the
-hand-written adjoint kernels; every day's record is kept where half of the free memory
-takes them, else the state is checkpointed every ``checkpoint_every`` days. ``calibrate`` fits theta to an observed daily-incidence curve with Adam on log(theta).
+hand-written adjoint kernels, with the state checkpointed every ``checkpoint_every`` days.
+Where the caller names no ``checkpoint_every``, every day's record is held instead (four values
+per agent and day, at most an eighth of the card's memory and half of what is free), which saves
+the backward a second forward. ``calibrate`` fits theta to an observed daily-incidence curve with
+Adam on log(theta).
 
 The per-agent relative transmissibility over time since infection,
 w_b(d) = E[infectious on lag d x viral load x asymptomatic factor], is tabulated per age
@@ -122,10 +125,18 @@ def age_bins(age, pars):
     return (np.digitize(np.asarray(age), pars['prognoses']['age_cutoffs']) - 1).astype(np.uint8)
 
 
-class Relaxation:
-    """Expected-infection relaxation of an initialized Sim (static layers, n_days days)."""
+class _Default(int):
+    """A default value, told by its type from an equal one that the caller gives."""
 
-    def __init__(self, sim, n_days=None, checkpoint_every=10, precision=32, w_samples=200_000, w_seed=0):
+
+class Relaxation:
+    """Expected-infection relaxation of an initialized Sim (static layers, n_days days).
+
+    ``checkpoint_every`` bounds the memory held: the records of that many days and one state per as many. Left at its
+    default, all days' records are held where they fit, and that many where they do not.
+    """
+
+    def __init__(self, sim, n_days=None, checkpoint_every=_Default(10), precision=32, w_samples=200_000, w_seed=0):
         import torch
         if not sim.initialized:
             sim.initialize()
@@ -154,6 +165,7 @@ class Relaxation:
         d.n_agents, d.n_layers, d.n_days = self.n, self.n_layers, self.n_days
         d.kernel_len = self.w.shape[1]
         d.checkpoint_every = int(checkpoint_every)
+        d.segment_days = _lib.RELAX_ALL_DAYS if isinstance(checkpoint_every, _Default) else 0
         d.precision = int(precision)
         d.seed_frac = self.seed_frac
         for li, lay in enumerate(self._csr):

@@ -815,11 +815,12 @@ typedef struct {
   int64_t n_agents;
   int32_t n_layers, n_days;
   int32_t kernel_len;          /* lags 0..kernel_len-1 of w_host per age bin */
-  int32_t checkpoint_every;    /* days between stored states where every day's record does not fit (the backward
-                                  then re-runs each segment) */
+  int32_t checkpoint_every;    /* days between stored states (the backward re-runs each segment) */
   int32_t precision;           /* 32 (float arithmetic) or 64 (double) */
-  int32_t segment_days;        /* 0: every day's record is held when half of the free memory takes them, else
-                                  checkpoint_every days; > 0: this many days. No result depends on it */
+  int32_t segment_days;        /* 1 .. n_days: in place of checkpoint_every; CVK_RELAX_ALL_DAYS: every day's record is
+                                  held (4 values per agent and day, and the backward re-runs nothing) where they take
+                                  at most an eighth of the card's memory and half of what is free; any other value:
+                                  checkpoint_every days. No result depends on it */
   double seed_frac;            /* pop_infected / n_agents */
   const int64_t* indptr[CVK_MAX_LAYERS];  /* device [n_agents + 1]: neighbour list offsets per layer (the lists
                                              are laid out anew at create and not read afterwards) */
@@ -830,6 +831,7 @@ typedef struct {
   double dyn_slots[CVK_MAX_LAYERS];  /* > 0: layer l is resampled every day and enters in expectation with
                                         this many contact slots per agent (indptr / nbr unused); 0: its lists */
 } cvk_relax_desc;
+#define CVK_RELAX_ALL_DAYS (-1)  /* segment_days */
 
 int cvk_relax_create(const cvk_relax_desc* desc, void** handle_out);
 int cvk_relax_destroy(void* handle);

@@ -407,6 +407,42 @@ def test_relax_ragged_lists_match_cpu_reference(gpu, n, precision):
 
 
 @pytest.mark.gpu
+def test_relax_memory_follows_checkpoint_every(gpu):
+    """A caller's checkpoint_every bounds what the handle holds; without one all days' records are held. A descriptor
+    whose segment_days is no length of a segment (0, or what a caller that does not know the field left there) is bound
+    by checkpoint_every too. The gradient is the same to the bit."""
+    import torch
+    from covasim_amd import _lib
+    from covasim_amd.relax import Relaxation
+    T = 60
+    sim = _sim(2 ** 18, T)  # a day's values take a whole allocation granule of 2 MiB
+
+    def free():  # outside torch's own pool
+        torch.cuda.synchronize()
+        return torch.cuda.mem_get_info()[0] + torch.cuda.memory_reserved()
+
+    def held(make):
+        before = free()
+        made = make()
+        return (before - free()) / (sim.people.n * 8), made  # in values per agent
+    slots = 50  # at most: 5 bytes for each contact of both directions, workgroup sums, and the granules of small arrays
+    make = lambda **kw: Relaxation(sim, precision=64, w_samples=2000, **kw)
+    rows, every = held(make)
+    assert rows >= 6 * T
+    theta, c = every.theta0() * 1.1, np.linspace(0.5, 1.5, T)
+    e, g = every.forward_np(theta), every.backward_np(theta, c)
+    for days in (5, 10):
+        rows, bound = held(lambda: make(checkpoint_every=days))
+        assert 2 * T <= rows <= 2 * T + 4 * days + T // days + 6 + slots, (days, rows)
+        assert np.array_equal(bound.forward_np(theta), e) and np.array_equal(bound.backward_np(theta, c), g)
+    for value, days in [(0, 10), (-7, 10), (T + 1, 10), (2 ** 31 - 1, 10), (3, 3), (_lib.RELAX_ALL_DAYS, T)]:
+        rows, h = held(lambda: _handle(every, segment_days=value))
+        assert rows <= 2 * T + 4 * days + -(-T // days) + 6 + slots, (value, rows)
+        got = _value_and_grad(h, theta, c)
+        assert np.array_equal(got[0], e) and np.array_equal(got[1], g), value
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize('precision', [32, 64])
 @pytest.mark.parametrize('n,lanes', [(0, 4), (200_000, 2)])  # four lanes share an agent's list, or two (n: at least)
 @pytest.mark.parametrize('x,counts', [(5.0, range(49, 57)), (0.9, range(304, 327)), (0.5, range(1018, 1080, 3))])
