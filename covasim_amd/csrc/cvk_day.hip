@@ -1225,14 +1225,23 @@ constexpr int32_t GRAPH_DAYS_FIRST = 4, GRAPH_DAYS_MAX = 32;
 
 static int run_days_graphs(const cvk_people* people, cvk_layer* layers, const cvk_params* params, cvk_work* work,
                            int32_t t0, int32_t t1, int64_t pop_infected, const cvk_imports* imports, hipStream_t st) {
-  // an import event that choose_impl would refuse is refused before any day has run
+  // What only a later part would refuse is refused before any day has run: an import event of a later day, and, where the
+  // dynamic layers' contacts are generated, the layers that the last day's close writes.
   for (int j = 0; imports && j < imports->n; ++j) {
     if (imports->days[j] < t0 || imports->days[j] >= t1) continue;
     const int rc = check_choose(people, params, imports->n_imports[j], CVK_LAYER_IMPORT, imports->variants[j]);
     if (rc) return rc;
   }
+  DayBeginArgs close;
+  memset(&close, 0, sizeof(close));
+  uint32_t close_blocks = 0;
+  int rc = fill_resample(close, layers, params, 1, &close_blocks);
+  if (rc) return rc;
+  const auto wait = [st, &rc]() {
+    if (hipStreamSynchronize(st) != hipSuccess && !rc) rc = fail(CVK_E_HIP, "cvk_run_days: device error");
+  };
   hipGraphExec_t parts[64];  // launched, not yet released
-  int n_parts = 0, rc = CVK_OK;
+  int n_parts = 0;
   uint32_t infect_blocks = 0;
   int32_t days = GRAPH_DAYS_FIRST;
   for (int32_t from = t0; from < t1 && !rc; from += days, days = std::min(2 * days, GRAPH_DAYS_MAX)) {
@@ -1243,11 +1252,11 @@ static int run_days_graphs(const cvk_people* people, cvk_layer* layers, const cv
     parts[n_parts++] = exec;
     if (hipGraphLaunch(exec, st) != hipSuccess) rc = fail(CVK_E_HIP, "cvk_run_days: hipGraphLaunch failed");
     if (n_parts == 64) {  // some 2000 days: release what has run
-      (void)hipStreamSynchronize(st);
+      wait();
       while (n_parts) (void)hipGraphExecDestroy(parts[--n_parts]);
     }
   }
-  (void)hipStreamSynchronize(st);
+  wait();
   while (n_parts) (void)hipGraphExecDestroy(parts[--n_parts]);
   return rc;
 }

@@ -520,7 +520,8 @@ int cvk_day_plan(const cvk_layer* layers, const cvk_params* params, const cvk_im
                  int32_t* out);
 /* Runs days [t0, t1) (t0 == 0 also seeds pop_infected infections first). use_graph != 0
  * captures the launches into hipGraphs of a few days each, launches each one once as soon as it is there, and waits
- * for the stream. */
+ * for the stream. A call refused for its arguments has run nothing then; after CVK_E_HIP (a later graph that could not
+ * be made, or an error of the device) some of the days may have run, and the state is to be restored. */
 int cvk_run_days(const cvk_people* people, cvk_layer* layers, const cvk_params* params, cvk_work* work,
                  int32_t t0, int32_t t1, int64_t pop_infected, const cvk_imports* imports,
                  int32_t use_graph, void* stream);

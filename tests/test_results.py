@@ -323,3 +323,54 @@ def test_import_refused_before_a_graph_run_starts():
     assert rc != 0
     after = sim.people.snapshot()
     assert all(np.array_equal(before[k], after[k], equal_nan=True) for k in before)
+
+
+@pytest.mark.gpu
+def test_layer_refused_before_a_graph_run_starts():
+    """A resampled layer whose weights the last day's close could not write (their address is no multiple of 8) is
+    refused before any day has run, also where no earlier day touches them (the contacts are generated)."""
+    import ctypes as C
+
+    import covasim_amd as cv
+    import torch
+    from covasim_amd import _lib
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        sim = cv.Sim(pop_size=2000, pop_type='hybrid', n_days=20, rand_seed=4, dynam_layer=dict(c=1))
+        sim.initialize()
+        torch.cuda.synchronize()
+        layers = type(sim._layers).from_buffer_copy(sim._layers)
+        index = sim.layer_keys().index('c')
+        assert layers[index].dynamic
+        layers[index].beta += 4
+        layers[index].n_edges -= 1
+        before = sim.people.snapshot()
+        _lib.check(_lib.lib().cvk_set_tuning(_lib.TUNE_GENERATE_DYNAMIC, 1), 'tuning')
+        try:
+            rc = _lib.lib().cvk_run_days(sim.people.struct(), layers, sim._params, sim._work, 0, sim.npts, 20,
+                                         C.byref(sim._imports), 1, C.c_void_p(stream.cuda_stream))
+        finally:
+            _lib.check(_lib.lib().cvk_set_tuning(_lib.TUNE_GENERATE_DYNAMIC, 2), 'tuning')
+        torch.cuda.synchronize()
+    assert rc == _lib.E_ALIGN
+    after = sim.people.snapshot()
+    assert all(np.array_equal(before[k], after[k], equal_nan=True) for k in before)
+
+
+@pytest.mark.gpu
+def test_more_graph_parts_than_are_kept_at_once():
+    """2100 days are 66 parts, the first 64 released while the run goes on: the results are an eager run's."""
+    import covasim_amd as cv
+    import torch
+
+    def run(graph):
+        sim = cv.Sim(pop_size=300, pop_type='hybrid', n_days=2100, rand_seed=4, beta=0.03, use_waning=True,
+                     dynam_layer=dict(c=1))
+        with torch.cuda.stream(torch.cuda.Stream() if graph else torch.cuda.current_stream()):
+            sim.run(use_graph=graph)
+        return sim
+    parts, eager = run(True), run(False)
+    for key, res in eager.results.items():
+        if key != 'variant':
+            assert np.array_equal(res.values, parts.results[key].values, equal_nan=True), key
+    assert eager.results['cum_reinfections'].values[-1] > 0
