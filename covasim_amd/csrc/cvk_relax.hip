@@ -55,6 +55,7 @@ constexpr int RELAX_MAX_PARAMS = 1 + CVK_MAX_LAYERS + RELAX_BINS;
 constexpr double RELAX_XMAX = 0.999999;  // per-edge probabilities are capped below 1 (1 - x stays positive)
 constexpr int RELAX_AB = 128;            // agents of a workgroup (64 for small populations)
 constexpr int RELAX_UNROLL = 8;          // neighbour-list entries of a lane whose gathers are in flight together
+constexpr int64_t RELAX_GROUP_SLOTS = (int64_t)1 << 31;  // most slots of a workgroup: its kernels count them in 32 bits
 constexpr int RELAX_LAGS = 64;           // lags of the infectiousness table staged in LDS together
 // packed slots: neighbour index, the held layer and the neighbour's age bin
 constexpr uint32_t RELAX_IDX = (1u << 25) - 1u;
@@ -887,7 +888,19 @@ struct Relax : RelaxBase {
     uint8_t *tgt = nullptr, *meta = nullptr;
     int rc = alloc(&base, (int64_t)D.n_blocks + 1);
     rc = rc ? rc : alloc(&tiles, scan_tiles(D.n_blocks) + 1);
-    rc = rc ? rc : alloc(&end, D.n);
+    rc = rc ? rc : scan(RelaxGroupSlots{L}, RelaxWriteBase{base}, (int64_t)D.n_blocks, tiles, base + D.n_blocks,
+                        (hipStream_t)nullptr);
+    if (rc) return rc;
+    if (total > RELAX_GROUP_SLOTS) {
+      std::vector<int64_t> first((size_t)D.n_blocks + 1);
+      if (hipMemcpy(first.data(), base, first.size() * sizeof(int64_t), hipMemcpyDeviceToHost) != hipSuccess)
+        return fail(CVK_E_HIP, "cvk_relax_create: cannot read the workgroups' offsets");
+      for (int32_t w = 0; w < D.n_blocks; ++w)
+        if (first[w + 1] - first[w] > RELAX_GROUP_SLOTS)
+          return failf(CVK_E_CAPACITY, "cvk_relax_create: agents %lld to %lld have more than 2^31 contact slots",
+                       (long long)w * ab, std::min((long long)D.n, (long long)(w + 1) * ab) - 1);
+    }
+    rc = alloc(&end, D.n);
     rc = rc ? rc : alloc(&slots, total);
     rc = rc ? rc : alloc(&tgt, total);
     if (D.n > (int64_t)RELAX_IDX + 1) rc = rc ? rc : alloc(&meta, total);
@@ -897,8 +910,6 @@ struct Relax : RelaxBase {
     D.slots = slots;
     D.meta = meta;
     D.tgt = tgt;
-    rc = scan(RelaxGroupSlots{L}, RelaxWriteBase{base}, (int64_t)D.n_blocks, tiles, base + D.n_blocks, (hipStream_t)nullptr);
-    if (rc) return rc;
     const auto fn = ab == 64 ? relax_layout_kernel<64> : relax_layout_kernel<RELAX_AB>;
     hipLaunchKernelGGL(fn, dim3(D.n_blocks), dim3(RELAX_BLOCK), 0, nullptr, L, D.bin, base, end, slots, meta, tgt);
     rc = check_launch("cvk_relax_create");

@@ -824,7 +824,8 @@ typedef struct {
                                   checkpoint_every days. No result depends on it */
   double seed_frac;            /* pop_infected / n_agents */
   const int64_t* indptr[CVK_MAX_LAYERS];  /* device [n_agents + 1]: neighbour list offsets per layer (the lists
-                                             are laid out anew at create and not read afterwards) */
+                                             are laid out anew at create and not read afterwards; CVK_E_CAPACITY
+                                             where 128 successive agents have more than 2^31 slots) */
   const int32_t* nbr[CVK_MAX_LAYERS];     /* device: both directions of every edge, no self-loops */
   const uint8_t* age_bin;      /* device [n_agents]: prognosis age bin 0..9 */
   const float* rel_trans;      /* device [n_agents] */

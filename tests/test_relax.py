@@ -490,6 +490,28 @@ def test_relax_escape_below_the_normal_doubles(gpu, precision, n, lanes, x, coun
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize('at', [0, 200])  # in the first workgroup, or a later one
+def test_relax_refuses_more_slots_than_a_workgroup_counts(gpu, at):
+    """Lists that claim 2^31 + 1 slots for one agent are refused from their offsets alone: no list is read."""
+    import ctypes as C
+    import torch
+    from covasim_amd import _lib
+    n, T = 300, 3
+    indptr = torch.zeros(n + 1, dtype=torch.int64, device='cuda')
+    indptr[at + 1:] = 2 ** 31 + 1
+    nbr = torch.zeros(4, dtype=torch.int32, device='cuda')
+    bins = torch.zeros(n, dtype=torch.uint8, device='cuda')
+    rt = torch.ones(n, device='cuda')
+    w = np.ones((10, T + 1))
+    d = _lib.RelaxDesc(n_agents=n, n_layers=1, n_days=T, kernel_len=T + 1, checkpoint_every=2, precision=32,
+                       seed_frac=0.1, age_bin=bins.data_ptr(), rel_trans=rt.data_ptr(), w_host=w.ctypes.data)
+    d.indptr[0], d.nbr[0] = indptr.data_ptr(), nbr.data_ptr()
+    h = C.c_void_p()
+    assert _lib.lib().cvk_relax_create(C.byref(d), C.byref(h)) == _lib.E_CAPACITY
+    assert not h.value and b'contact slots' in _lib.lib().cvk_last_error()
+
+
+@pytest.mark.gpu
 def test_relax_more_agents_than_a_packed_slot_addresses(gpu):
     """2^25 + 3 agents (a slot's layer and bin then travel beside its index), contacts among the last few only: the
     expected infections and gradient are those of the same few agents alone."""
