@@ -51,7 +51,7 @@ WORKLOADS = {
                     pars=dict(beta=0.016, use_waning=False, pop_infected=20, dynam_layer=dict(c=1)),
                     desc='differentiable relaxation on the hybrid 1M population (h/s/w held, c resampled daily '
                          'and taken in expectation), 60 days: '
-                         'float32 forward + hand-written adjoint with checkpoints every 10 days, gradient wrt '
+                         'float32 forward + hand-written adjoint with the records of every day held, gradient wrt '
                          '4 layer betas, beta and 10 age-bin rel_sus; calibration to a stochastic incidence curve'),
     'interv1m': dict(pop_size=1_000_000, pop_type='hybrid', n_days=180, households='categorical', interventions=True,
                      pars=dict(beta=0.016, use_waning=False, pop_infected=20, dynam_layer=dict(c=1)),
@@ -417,11 +417,12 @@ def run_relax(w, args):
     # counted): per day t a forward (relax_day_kernel: bin, rel_trans, s read and written, the end of the agent's
     # list, delta, tr and the day's three records written, min(t, kmax) past deltas, 4 per neighbour slot) and the
     # adjoint (relax_adjoint_kernel: bin, rel_trans, the list's end, the three records, tr of two days, lbar and
-    # sbar read and written, ibar written, min(kmax, T-1-t) ibar rows, 4 per slot)
+    # sbar read and written, ibar and the neighbours' input written, min(kmax, T-1-t) ibar rows, 5 per slot: its word
+    # and its owner's byte)
     slots = int(sum(lay[1].numel() for lay in r32._csr if lay is not None))
     kmax = min(r32.w.shape[1] - 1, T)
     fwd = sum(n * (37 + 4 * min(t, kmax)) + 4 * slots for t in range(T))
-    adj = sum(n * (49 + 4 * min(kmax, T - 1 - t)) + 4 * slots for t in range(T))
+    adj = sum(n * (53 + 4 * min(kmax, T - 1 - t)) + 5 * slots for t in range(T))
     fb_bytes = fwd + adj
     fb_gbs = fb_bytes / fb_ev_s / 1e9
     out = {

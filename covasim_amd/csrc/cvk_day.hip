@@ -531,10 +531,12 @@ static int g_edge_lds = 1;     // tunable: stage the infectious bitmap in LDS wh
 static int g_edge_chunks = 2;  // tunable: 4-edge chunks per lane per wave tile (2 or 4)
 static int g_gen_dynamic = 2;  // tunable: the fused day loop computes dynamic layers' endpoints in place
                                // (1), writes each day's resample (0), or chooses by size (2)
-// Auto choice: writing a day's resample of E dynamic edges costs 8E bytes of stores inside the
-// latency-bound infect pass, generating them costs E/2 Philox blocks in the edge and infect passes.
-// Measured: 10M dynamic edges (hybrid 1M) 0.092 ms/day writing against 0.097 generating; 100M
-// (hybrid 10M) 1.70 against 1.48. Generation is chosen from 2^25 dynamic edges up.
+// Auto choice: writing a day's resample of E dynamic edges costs 8E bytes of stores inside the infect pass and as many
+// read by the edge pass, generating them E/2 Philox blocks in the edge and infect passes. Whole runs, writing ->
+// generating: equal at 0.5M to 0.7M dynamic edges; 5M (500k agents, 46 days, with the script around them) 8.9 -> 8.4 ms;
+// 10M (hybrid 1M, 181 days) 16.4 -> 15.4 ms; 100M (hybrid 10M) 1.70 -> 1.48 ms a day. The line at 2^25 is the documented
+// meaning of the tunable's value 2, from when 10M took 0.092 ms a day written and 0.097 generated; value 1 generates at
+// every size.
 constexpr int64_t GEN_AUTO_MIN_EDGES = (int64_t)1 << 25;
 static int g_source_lists = 2;   // tunable: walk static layers through their source lists when given:
                                  // 0 never, 1 always, 2 on days with few infectious agents (g_source_permille)

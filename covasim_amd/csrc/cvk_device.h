@@ -64,7 +64,7 @@ struct u32x4 {
 
 // a ^ b ^ c; on the device one v_bitop3_b32 (the compiler emits two v_xor_b32), so a Philox round is two 32 x 32 -> 64
 // multiplies and two of these. Whole runs bound by the generator (contacts resampled or generated each day): 1M agents
-// x 120 days 16.7 -> 16.3 ms, 64 sims of a batch 95.3 -> 93.7 ms, 10M agents 152.4 -> 151.1 ms.
+// x 180 days 16.7 -> 16.3 ms, 64 sims of a batch 95.3 -> 93.7 ms, 10M agents 152.4 -> 151.1 ms.
 __host__ __device__ inline uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
 #if defined(__HIP_DEVICE_COMPILE__)
   return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);

@@ -304,7 +304,7 @@ struct AgentSpan {
 // bytes on quiet days); otherwise every field is loaded in one round trip.
 // sev: compute and store sev_imm too. Else the day's infect pass computes it for its targets (infect_sev_imm); its
 // only other reader is the state after the run's last day. A third of the pass's powers, which bound it late in a run
-// with waning: 10M agents x 60 days 152.4 -> 150.3 ms. The batched pass always stores: there the powers hide behind
+// with waning: 10M agents x 120 days 152.4 -> 150.3 ms. The batched pass always stores: there the powers hide behind
 // the loads, and its infect pass, with many more targets a day, took longer by them (95.3 -> 95.9 ms).
 template <int APT, bool LAZY>
 __device__ void agent_block(const cvk_people& P, const cvk_params& prm, const AgentSpan& S, int32_t t,

@@ -51,7 +51,6 @@ namespace cvk {
 
 constexpr int RELAX_BLOCK = 256;
 constexpr int RELAX_BINS = 10;
-constexpr int RELAX_MAX_PARAMS = 1 + CVK_MAX_LAYERS + RELAX_BINS;
 constexpr double RELAX_XMAX = 0.999999;  // per-edge probabilities are capped below 1 (1 - x stays positive)
 constexpr int RELAX_AB = 128;            // agents of a workgroup (64 for small populations)
 constexpr int RELAX_UNROLL = 8;          // neighbour-list entries of a lane whose gathers are in flight together

@@ -9,8 +9,8 @@
 ``Relaxation.expected(theta)`` returns the expected new infections of each day, E_t, as
 a differentiable torch function of theta = [beta, beta_layer for each layer, rel_sus for
 the 10 prognosis age bins]. The model and its adjoint are spelled out in
-``csrc/cvk_relax.hip``. The forward runs in float32 (precision=32, log-space products
-accumulated in float32) or float64 (precision=64). The gradient comes from the
+``csrc/cvk_relax.hip``. It runs in float32 (precision=32, with the escape products, and every sum
+beyond one agent's lags or one thread's contacts, in float64) or float64 (precision=64). The gradient comes from the
 hand-written adjoint kernels, with the state checkpointed every ``checkpoint_every`` days.
 Where the caller names no ``checkpoint_every``, every day's record is held instead (four values
 per agent and day, at most an eighth of the card's memory and half of what is free), which saves
