@@ -117,11 +117,14 @@ def compute_infections(beta, p1, p2, layer_betas, rel_trans, rel_sus, legacy=Fal
         raise IndexError('contact indices outside [0, len(rel_trans))')
     u = None
     if uniforms is not None:
-        u, _ = _dev(uniforms, np.float64, 'uniforms')
-        if u.numel() != 2 * E:
+        try:
+            u, _ = _dev(uniforms, np.float64, 'uniforms')
+            if u.numel() != 2 * E:
+                raise ValueError('uniforms must have shape (2, n_edges)')
+        except (TypeError, ValueError):  # an index outside the population is what is reported, as without uniforms
             if E and (int(torch.minimum(a1.min(), a2.min())) < 0 or int(torch.maximum(a1.max(), a2.max())) >= n):
-                raise IndexError('contact indices outside [0, len(rel_trans))')
-            raise ValueError('uniforms must have shape (2, n_edges)')
+                raise IndexError('contact indices outside [0, len(rel_trans))') from None
+            raise
     cap = (E if legacy else 2 * E)
     src = torch.empty(max(cap, 1), dtype=torch.int32, device=a1.device)
     tgt = torch.empty(max(cap, 1), dtype=torch.int32, device=a1.device)

@@ -162,6 +162,17 @@ def test_infections_of_no_agents(gpu, host):
     assert [len(x) for x in cv.utils.compute_infections(0.3, ends, ends, nobody, nobody, nobody)] == [0, 0]
 
 
+def test_infections_report_the_index_before_the_uniforms(gpu):
+    """Uniforms of the wrong shape or type are refused as such, unless an index is outside the population too."""
+    import covasim_amd as cv
+    p, one, factor = np.zeros(3, np.int32), np.ones(3, np.float32), np.ones(5, np.float32)
+    for uniforms, error in [(np.zeros((1, 3)), ValueError), (np.zeros((2, 3), np.float32), TypeError)]:
+        with pytest.raises(error):
+            cv.utils.compute_infections(0.3, p, p, one, factor, factor, uniforms=uniforms)
+        with pytest.raises(IndexError):
+            cv.utils.compute_infections(0.3, p + 5, p, one, factor, factor, uniforms=uniforms)
+
+
 def test_infections_of_more_agents_than_32_bits_count(gpu):
     """2^32 + 5 agents: an index is checked against all of them (a negative one is still refused), and the infections
     are those among the agents that the contacts name."""
