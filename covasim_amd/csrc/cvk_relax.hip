@@ -507,7 +507,8 @@ __global__ __launch_bounds__(RELAX_BLOCK) void relax_adjoint_kernel(RelaxDev<R> 
           if (e < cn) {
             const uint32_t h = m[u] & 7u;
             const R rate = s_rate[h], tra = s_tra[aa[u]];
-            const R term = y[u] * relax_gp<R>((rate * s_sig[m[u] >> 4]) * tra, xmax);  // a -> j
+            const R x = (rate * s_sig[m[u] >> 4]) * tra;  // a -> j
+            const R term = x < xmax ? y[u] * relax_rcp(x - (R)1) : (R)0;  // (y: 0 * inf for an infinite sigma)
             stage[e] = rate * term;
             s_g[h * RELAX_BLOCK + threadIdx.x] += tra * term;
           }

@@ -490,6 +490,30 @@ def test_relax_escape_below_the_normal_doubles(gpu, precision, n, lanes, x, coun
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize('precision', [32, 64])
+def test_relax_a_bin_that_never_escapes(gpu, precision):
+    """An infinite sigma saturates every contact of its bin: its own derivative is zero, and the others are those of
+    float64 central differences (step h = 1e-4 relative, whose error is of the order of h^2)."""
+    from covasim_amd.relax import Relaxation
+    sim = _sim(600, 20)
+    relax, r64 = (Relaxation(sim, precision=p, w_samples=5000) for p in (precision, 64))
+    theta = relax.theta0() * np.linspace(0.8, 1.2, relax.n_params)
+    forever = 1 + relax.n_layers + 4
+    theta[0], theta[forever] = 0.1, np.inf
+    assert (relax.bins_np == 4).sum() > 20
+    c = np.random.default_rng(4).uniform(0.5, 1.5, relax.n_days)
+    assert _rel(relax.forward_np(theta), r64.forward_np(theta)) <= 100 * 2.0 ** -24
+    got, want, h = relax.backward_np(theta, c), np.zeros(relax.n_params), 1e-4
+    for k in set(range(relax.n_params)) - {forever}:
+        up, down = theta.copy(), theta.copy()
+        up[k] *= 1 + h
+        down[k] *= 1 - h
+        want[k] = (c @ r64.forward_np(up) - c @ r64.forward_np(down)) / (2 * h * theta[k])
+    assert np.linalg.norm(want) > 0
+    assert _rel(got, want) <= 1e-4
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize('at', [0, 200])  # in the first workgroup, or a later one
 def test_relax_refuses_more_slots_than_a_workgroup_counts(gpu, at):
     """Lists that claim 2^31 + 1 slots for one agent are refused from their offsets alone: no list is read."""
