@@ -70,7 +70,7 @@ __global__ void trans_sus_kernel(const float* __restrict__ rel_trans, const floa
 // bit lookups at 10M edges, the bitmap in LDS up to ~1.1M agents); before, both a counting and a writing pass
 // gathered rel_trans at both ends of every edge and drew a Philox block per slot with a nonzero source, with one
 // workgroup scanning the counts between them: 129 + 149 + 21 us at 1M agents and 10M edges, 5 % of them
-// infectious, against 4 + 50 + 15 us. (The next chunk's columns loaded ahead of the candidates: 55 us.)
+// infectious, against 4 + 50 + 12 us. (The next chunk's columns loaded ahead of the candidates: 55 us.)
 // cvk_infections_noalloc, whose scratch is fixed, keeps the waves' counts and a flag for each chunk: its writing pass
 // finds the hits of the flagged chunks anew (213 us at the sizes above with 4050 pairs; 181 with a hit bit for
 // every slot, which took 16 MiB of every process on every GPU; 302 without the flags).
